@@ -44,7 +44,7 @@ HIP_FLAGS = [
 #   decode 44.2 -> 39.8 us, ragged B64 decode 104 -> 102.4 us on MI355X.
 VGPR_MFMA = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 HIP_FILE_FLAGS = {"prefill_fa.hip": ["-fno-honor-nans"], "prefill_ext.hip": ["-fno-honor-nans"],
-                  "decode_splitkv.hip": VGPR_MFMA,
+                  "decode_splitkv.hip": VGPR_MFMA, "quant_matmul.hip": VGPR_MFMA,
                   "peak_probe.hip": VGPR_MFMA}
 C_FLAGS = ["-std=c11", "-O2", "-fPIC", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__",
            f"-I{ROCM}/include", f"-I{CSRC}", f"-I{INCLUDE}"]

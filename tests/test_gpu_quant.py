@@ -216,3 +216,67 @@ def test_q4_0_q8_0_reference_patterns(gpu, orc, qtype):
     out = la.DeviceArray.zeros((1, n_rows), np.float32)
     la.matmul_prequant(out, dev(la, w), qtype, n_rows, n_cols, dev(la, xq), 1)
     assert np.array_equal(out.numpy().view(np.uint32), orc.matmul_q(w, qtype, xq, n_cols).view(np.uint32))
+
+
+@pytest.mark.parametrize("qtype", [2, 8, 12, 13, 14, 23])
+@pytest.mark.parametrize("n_rows,n_cols,B", [(5, 768, 5),         # few tokens: one ragged 16 x 16 tile
+                                             (1000, 768, 270),    # 64-row x 32-token tiles, both ragged
+                                             (2050, 256, 260),    # x 64 tokens
+                                             (2060, 512, 1030)])  # x 128 tokens
+def test_matrix_pipe_tiles_bit_exact(gpu, orc, qtype, n_rows, n_cols, B):
+    """Every tile shape of the matrix-pipe product, rows and tokens past the
+    last tile's edge, a zero activation block and activations at -128; tokens
+    around every tile edge against the oracle."""
+    la = gpu
+    rng = np.random.default_rng(qtype * 100 + n_rows + B)
+    w = q_random(rng, qtype, n_rows, n_cols)
+    x = rng.standard_normal((B, n_cols)).astype(np.float32)
+    x[0, :256] = 0.0
+    xq = orc.quantize_q8_K(x)
+    xq[1, 4:260] = 128  # int8 -128 throughout, bsums to match
+    xq[1, 260:292] = np.full(16, -2048, np.int16).view(np.uint8)
+    out = la.DeviceArray.zeros((B, n_rows), np.float32)
+    la.matmul_prequant(out, dev(la, w), qtype, n_rows, n_cols, dev(la, xq), B)
+    pick = sorted({t for e in range(0, B + 1, 16) for t in (e - 1, e) if 0 <= t < B} | {1, B - 1})
+    want = orc.matmul_q(w, qtype, np.ascontiguousarray(xq[pick]), n_cols)
+    assert np.array_equal(out.numpy()[pick].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("types", [[12, 12, 14], [13, 8, 23, 2]])
+def test_matrix_pipe_mixed_set(gpu, orc, types):
+    """A set of several types in one matrix-pipe launch (128-token tiles, and
+    64-token tiles when Q4_0 is in the set)."""
+    la = gpu
+    rng = np.random.default_rng(sum(types))
+    n_cols, rows, B = 512, [1100, 520, 500, 16][:len(types)], 1030
+    ws = [q_random(rng, t, r, n_cols) for t, r in zip(types, rows)]
+    xq = orc.quantize_q8_K(rng.standard_normal((B, n_cols)).astype(np.float32))
+    outs = [la.DeviceArray.zeros((B, r), np.float32) for r in rows]
+    la.gqa_qkv_fused(outs, [dev(la, w) for w in ws], types, rows, n_cols, dev(la, xq), B)
+    pick = [0, 15, 16, 127, 128, 500, 1023, 1024, 1029]
+    for o, w, t in zip(outs, ws, types):
+        want = orc.matmul_q(w, t, np.ascontiguousarray(xq[pick]), n_cols)
+        assert np.array_equal(o.numpy()[pick].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("qtype", [2, 8, 12, 13, 14, 23])
+@pytest.mark.parametrize("n_rows,B", [(20, 6), (1000, 270)])
+def test_matrix_pipe_row_scale_not_finite(gpu, orc, qtype, n_rows, B):
+    """Rows whose fp16 scale is infinite: a zero activation block is left out
+    (its product with the scale would be NaN), others give the reference's
+    infinities and NaN; the rows beside them are untouched."""
+    la = gpu
+    rng = np.random.default_rng(qtype + B)
+    n_cols = 512
+    w = q_random(rng, qtype, n_rows, n_cols)
+    at = 208 if qtype == 14 else 0
+    w[3, at:at + 2] = np.array([0x7C00], np.uint16).view(np.uint8)
+    x = rng.standard_normal((B, n_cols)).astype(np.float32)
+    x[::2, :256] = 0.0
+    xq = orc.quantize_q8_K(x)
+    out = la.DeviceArray.zeros((B, n_rows), np.float32)
+    la.matmul_prequant(out, dev(la, w), qtype, n_rows, n_cols, dev(la, xq), B)
+    pick = list(range(min(B, 40)))
+    want = orc.matmul_q(w, qtype, np.ascontiguousarray(xq[pick]), n_cols)
+    assert np.array_equal(out.numpy()[pick], want, equal_nan=True)
+    assert np.isfinite(want[::2, 3]).all()
