@@ -96,3 +96,37 @@ def test_qkv_prologue_batched(gpu, orc):
             wk = orc.qk_norm_rope(k[s, r], nkv, hd, kw, eps, cos[p], sin[p], store_f16=True)
             assert np.array_equal(ks[slot].reshape(-1), wk), f"k s={s} r={r}"
             assert np.array_equal(vs[slot].reshape(-1), f16(v[s, r]).reshape(-1))
+
+
+@pytest.mark.parametrize("hd,table", [(64, False), (64, True), (128, False), (128, True)])
+@pytest.mark.parametrize("nq,nkv,norm", [(3, 1, True), (32, 8, True), (16, 4, False), (7, 7, True)])
+def test_qkv_prologue_head_groups(gpu, orc, hd, table, nq, nkv, norm):
+    """8 heads of a row per wave: groups that end inside the query heads, hold
+    both kinds, or run past the last KV head; several rows and sequences, ring
+    slots, every row bit for bit against the oracle."""
+    la = gpu
+    rng = np.random.default_rng(hd + nq + table)
+    n_seq, rows, win, cap, eps = 2, 5, 4, 9, 1e-5
+    cos, sin = la.rope_table_lfm2(64, hd, 1e6)
+    pos0 = np.array([3, 40], np.uint32)
+    q = rng.standard_normal((n_seq, rows, nq, hd), dtype=np.float32) * 2
+    k = rng.standard_normal((n_seq, rows, nkv, hd), dtype=np.float32) * 2
+    v = rng.standard_normal((n_seq, rows, nkv, hd), dtype=np.float32)
+    qw, kw = ((1 + 0.05 * rng.standard_normal(hd)).astype(np.float32) if norm else None for _ in range(2))
+    kd = [la.DeviceArray.zeros((cap, nkv, hd), np.uint16) for _ in range(n_seq)]
+    vd = [la.DeviceArray.zeros((cap, nkv, hd), np.uint16) for _ in range(n_seq)]
+    qd = dev(la, q)
+    la.qkv_prologue(qd, dev(la, k), dev(la, v), la.pointer_table(kd), la.pointer_table(vd), dev(la, pos0), n_seq, rows,
+                    nq, nkv, hd, None if qw is None else dev(la, qw), None if kw is None else dev(la, kw), eps,
+                    dev(la, cos), dev(la, sin), win, cap,
+                    prologue=la.PROLOGUE_TABLE if table else la.PROLOGUE_FAST)
+    got = qd.numpy()
+    for s in range(n_seq):
+        kc, vc = kd[s].numpy(), vd[s].numpy()
+        for r in range(rows):
+            p = int(pos0[s]) + r
+            want = orc.qk_norm_rope(q[s, r].ravel(), nq, hd, qw, eps, cos[p], sin[p], table=table)
+            assert np.array_equal(got[s, r].ravel().view(np.uint32), want.view(np.uint32)), (s, r)
+            want = orc.qk_norm_rope(k[s, r].ravel(), nkv, hd, kw, eps, cos[p], sin[p], store_f16=True, table=table)
+            assert np.array_equal(kc[p % cap].ravel(), want), (s, r)
+            assert np.array_equal(vc[p % cap].ravel(), v[s, r].astype(np.float16).view(np.uint16).ravel()), (s, r)
