@@ -155,6 +155,25 @@ __device__ __forceinline__ float gate_apply(float raw, const float *gate, int is
     return (gate && is_logit) ? 1.0f / (1.0f + expf(-raw)) : raw;
 }
 
+/* x of the lane 32 (16) further or back, both halves (row pairs) of the wave at
+ * once: lo = the value of the lower of the two lanes, hi = of the upper one, on
+ * both.  One VALU instruction where a shuffle goes through the LDS unit. */
+struct LanePair {
+    float lo, hi;
+};
+__device__ __forceinline__ LanePair pair32(float x) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, x);
+    const auto r     = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    const uint32_t lo = r[0], hi = r[1];
+    return {__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
+}
+__device__ __forceinline__ LanePair pair16(float x) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, x);
+    const auto r     = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const uint32_t lo = r[0], hi = r[1];
+    return {__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
+}
+
 /* Sum of squares of one head held in MFMA fragment order (lane (l16, g)
  * holds dims 32*st + 8*g + j), added in the order of the reference's AVX2
  * kernels so the normalised rows are bit-identical to theirs; the result is
@@ -166,10 +185,11 @@ __device__ __forceinline__ float gate_apply(float raw, const float *gate, int is
  *   HD 128 (lfm3_qk_norm_rope_128_avx2, tools/lfm3_engine.c:480-494): per
  *   column j, fma chains ss0 over dims 16k + j and ss1 over 16k + 8 + j,
  *   k = 0..7, s[j] = ss0 + ss1, then ((s0+s4) + (s1+s5)) + ((s2+s6) + (s3+s7)).
- * Dims 16k + j alternate between lanes g and g + 2, so the chains hop
- * between the two halves of the wave. */
+ * Dims 16k + j alternate between lanes g and g + 2: at 128 each lane takes its
+ * partner's dims too and runs the whole chain (passing the chain from half to
+ * half took 72 dependent shuffles). */
 template <int HD>
-__device__ __forceinline__ float sumsq_ref_order(const float (&x)[HD / 32][8], int g) {
+__device__ __forceinline__ float sumsq_ref_order(const float (&x)[HD / 32][8]) {
 #pragma clang fp contract(off)
     float t[8];
     if constexpr (HD == 64) {
@@ -177,31 +197,26 @@ __device__ __forceinline__ float sumsq_ref_order(const float (&x)[HD / 32][8], i
         for (int j = 0; j < 8; ++j) {
             const float a = x[0][j], b = x[1][j];
             const float v = a * a + b * b;                    /* g 0: ss0, g 1: ss1 (first terms) */
-            const float w = __shfl_xor(v, 32);                /* to g 2 / g 3                     */
-            const float u = __builtin_fmaf(a, a, __builtin_fmaf(b, b, w)); /* g 2: ss0, g 3: ss1 */
-            t[j]          = u + __shfl_xor(u, 16);            /* g 2, 3: ss0 + ss1                */
+            const float u = __builtin_fmaf(a, a, __builtin_fmaf(b, b, pair32(v).lo)); /* g 2: ss0, g 3: ss1 */
+            const LanePair q = pair16(u);
+            t[j]             = q.lo + q.hi;                   /* g 2, 3: ss0 + ss1                */
         }
         const float T = ((t[0] + t[4]) + (t[2] + t[6])) + ((t[1] + t[5]) + (t[3] + t[7]));
-        const float o = __shfl_xor(T, 32);
-        return g >= 2 ? T : o;
+        return pair32(T).hi;
     } else {
         static_assert(HD == 128, "reference summation order is defined for head_dim 64 and 128");
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             float acc = 0.0f;
 #pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                const float xx = x[st][j];
-                if (g < 2) acc = __builtin_fmaf(xx, xx, acc); /* dims 32 st + j (+8)        */
-                acc = __shfl_xor(acc, 32);
-                if (g >= 2) acc = __builtin_fmaf(xx, xx, acc); /* dims 32 st + 16 + j (+8)  */
-                acc = __shfl_xor(acc, 32);
+            for (int st = 0; st < 4; ++st) { /* dims 32 st + j (+8), then 32 st + 16 + j (+8) */
+                const LanePair p = pair32(x[st][j]);
+                acc              = __builtin_fmaf(p.hi, p.hi, __builtin_fmaf(p.lo, p.lo, acc));
             }
-            t[j] = acc + __shfl_xor(acc, 16); /* g 0, 1: ss0 + ss1 */
+            const LanePair q = pair16(acc);
+            t[j]             = q.lo + q.hi; /* ss0 + ss1 */
         }
-        const float T = ((t[0] + t[4]) + (t[1] + t[5])) + ((t[2] + t[6]) + (t[3] + t[7]));
-        const float o = __shfl_xor(T, 32);
-        return g < 2 ? T : o;
+        return ((t[0] + t[4]) + (t[1] + t[5])) + ((t[2] + t[6]) + (t[3] + t[7]));
     }
 }
 
@@ -248,36 +263,44 @@ __device__ __forceinline__ void load8(const float *p, float (&x)[8]) {
     x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
 }
 
-template <int HD>
+template <int HD, typename F>
 __device__ __forceinline__ void norm_rope_frag(float (&x)[HD / 32][8], uint32_t pos, const float *norm_w, float eps,
-                                               const float *cos_lut, const float *sin_lut, int g, int prologue) {
+                                               const float *cos_lut, const float *sin_lut, int g, int prologue,
+                                               const F &issue) {
     constexpr int NS = HD / 32, HALF = HD / 2;
-    if (norm_w) {
-        const float mean = prologue == LFM_PROLOGUE_TABLE ? meansq_table_order<HD>(x, (int)(threadIdx.x & 15u))
-                                                          : sumsq_ref_order<HD>(x, g) / (float)HD;
-        const float irms = 1.0f / sqrtf(mean + eps);
-#pragma unroll
-        for (int st = 0; st < NS; ++st) {
-            float w[8];
-            load8(norm_w + 32 * st + 8 * g, w);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) x[st][j] = (x[st][j] * irms) * w[j];
-        }
-    }
+    /* every load before the first use of x: one memory round trip, not three;
+     * then issue() adds loads of the caller's, which the sums do not wait for */
+    float c[NS / 2][8], sn[NS / 2][8], w[NS][8];
     const float *cr = cos_lut + (size_t)pos * HALF;
     const float *sr = sin_lut + (size_t)pos * HALF;
 #pragma unroll
     for (int st = 0; st < NS / 2; ++st) {
-        float c[8], sn[8];
-        load8(cr + 32 * st + 8 * g, c);
-        load8(sr + 32 * st + 8 * g, sn);
+        load8(cr + 32 * st + 8 * g, c[st]);
+        load8(sr + 32 * st + 8 * g, sn[st]);
+    }
+    if (norm_w)
+#pragma unroll
+        for (int st = 0; st < NS; ++st) load8(norm_w + 32 * st + 8 * g, w[st]);
+    __builtin_amdgcn_sched_barrier(0);
+    issue();
+    __builtin_amdgcn_sched_barrier(0);
+    if (norm_w) {
+        const float mean = prologue == LFM_PROLOGUE_TABLE ? meansq_table_order<HD>(x, (int)(threadIdx.x & 15u))
+                                                          : sumsq_ref_order<HD>(x) / (float)HD;
+        const float irms = 1.0f / sqrtf(mean + eps);
+#pragma unroll
+        for (int st = 0; st < NS; ++st)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[st][j] = (x[st][j] * irms) * w[st][j];
+    }
+#pragma unroll
+    for (int st = 0; st < NS / 2; ++st)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const float lo = x[st][j], hi = x[st + NS / 2][j];
-            x[st][j]          = __builtin_fmaf(lo, c[j], -(hi * sn[j]));
-            x[st + NS / 2][j] = __builtin_fmaf(hi, c[j], lo * sn[j]);
+            x[st][j]          = __builtin_fmaf(lo, c[st][j], -(hi * sn[st][j]));
+            x[st + NS / 2][j] = __builtin_fmaf(hi, c[st][j], lo * sn[st][j]);
         }
-    }
 }
 
 /* Two fp32 values stored as RNE fp16 (packed).  Each value is first
@@ -400,7 +423,12 @@ __device__ __forceinline__ void run_segment(const SplitParams &P, uint16_t *vt, 
     /* the first sub-tile is in flight while the query fragments are built */
     const uint32_t nsub = (ke - kb + 31u) / 32u;
     u32x4_t kA[2][NS], vA[NVL], kB[2][NS], vB[NVL];
-    load_tile(kb, kA, vA, false);
+    /* with the fused prologue and one query tile: right behind the loads of Q
+     * and its prologue, whose sums then run while it is in flight (loads
+     * complete in order; window step 12.4 -> 11.8 us, LFM3 B32 x 32768 342.7 ->
+     * 340.2) */
+    constexpr bool LATE = FUSE && NT == 1;
+    if constexpr (!LATE) load_tile(kb, kA, vA, false);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) koffb[kt] = (uint32_t)(((16 * kt + l16) * row + 8 * g) * sizeof(uint16_t));
 #pragma unroll
@@ -409,6 +437,45 @@ __device__ __forceinline__ void run_segment(const SplitParams &P, uint16_t *vt, 
         for (int i = 0; i < 4; ++i)
             voffb[ps * 4 + i] =
                 (uint32_t)(((4 * (ps * QPP + lane / CH) + i) * row + 8 * (lane % CH)) * sizeof(uint16_t));
+
+    /* ---- fused prologue: the rows of this call's positions -------------------
+     * Keys >= pos0 are the new tokens.  Before the key loop, the wave whose
+     * range [kb, ke) holds new keys builds those rows from the raw k/v
+     * (normalised, rotated, RNE fp16), stores them at their cache slots and
+     * stages them in its LDS area `fresh` ([n_rows][HD] K, then V).  Each new
+     * key lies in exactly one segment of the plan, so each row is stored once,
+     * and no other wave reads those bytes in this launch.  In the loop, the
+     * sub-tiles that reach pos0 take those rows from LDS in place of what was
+     * loaded from the slots (lanes clamped past ke take the last key's row
+     * too, so no stale slot content enters the product); the loop itself
+     * issues no extra global memory operations.
+     * Where they fit (one query tile, as in decode), the new key rows r0..r1-1
+     * take the tile's columns past the queries, so that one pass of loads, sums
+     * and rotations serves both (LFM3 window step B32 14.1 -> 12.4 us, ragged B64 97.1 ->
+     * 94.8; the separate pass took 2.6 us of each workgroup that has one). */
+    const bool has_fresh = FUSE && ke > pos0;
+    const uint32_t r0 = has_fresh ? max(kb, pos0) - pos0 : 0u, r1 = has_fresh ? ke - pos0 : 0u;
+    const bool spare = FUSE && NT == 1 && has_fresh && P.ncols + (r1 - r0) <= 16u && !P.q_norm_w == !P.k_norm_w;
+    uint16_t *kw = nullptr, *vw = nullptr; /* the cache rows, to be written */
+    float vraw[8];                         /* this lane's first piece of the new value rows */
+    if constexpr (FUSE) {
+        if (has_fresh) {
+            kw = const_cast<uint16_t *>(P.k_seq ? P.k_seq[s] : P.k_base + (size_t)s * P.seq_stride) + (size_t)kvh * HD;
+            vw = const_cast<uint16_t *>(P.v_seq ? P.v_seq[s] : P.v_base + (size_t)s * P.seq_stride) + (size_t)kvh * HD;
+            const uint32_t e = r0 * CH + (uint32_t)lane;
+            if (e < r1 * CH) load8(P.v_new + (((size_t)s * P.n_rows + e / CH) * P.n_head_kv + kvh) * HD + 8 * (e % CH), vraw);
+        }
+    }
+    /* one normalised, rotated key row (this lane's dims) to its slot and the LDS area */
+    auto put_key = [&](uint32_t r, const float (&x)[NS][8]) {
+        const size_t off = (size_t)lfm_slot_of(pos0 + r, P.window, P.cap) * row + 8 * g;
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            const u32x4_t w = pack8_rne(x[st]);
+            *reinterpret_cast<u32x4_t *>(kw + off + 32 * st)                       = w;
+            *reinterpret_cast<u32x4_t *>(fresh + (size_t)r * HD + 8 * g + 32 * st) = w;
+        }
+    };
 
     /* ---- per-column row bounds and Q fragments ------------------------------ */
     uint32_t col_lo[NT], col_hi[NT];
@@ -420,8 +487,15 @@ __device__ __forceinline__ void run_segment(const SplitParams &P, uint16_t *vt, 
         col_hi[nt] = 0u;
         float x[NS][8];
         const bool live = n < P.ncols;
+        const bool key  = spare && !live && n < P.ncols + (r1 - r0); /* a new key row in a spare column */
         uint32_t abs    = pos0;
-        if (live) {
+        if (key) {
+            const uint32_t r = r0 + n - P.ncols;
+            abs              = pos0 + r;
+            const float *kp  = P.k_new + (((size_t)s * P.n_rows + r) * P.n_head_kv + kvh) * HD + 8 * g;
+#pragma unroll
+            for (int st = 0; st < NS; ++st) load8(kp + 32 * st, x[st]);
+        } else if (live) {
             const uint32_t r = n / P.kv_mul;
             const uint32_t h = kvh * P.kv_mul + (n - r * P.kv_mul);
             abs              = pos0 + r;
@@ -438,7 +512,17 @@ __device__ __forceinline__ void run_segment(const SplitParams &P, uint16_t *vt, 
         }
         /* fused prologue: the raw query is normalised and rotated here, by
          * every wave that reads it (all lanes take part in the sums) */
-        if constexpr (FUSE) norm_rope_frag<HD>(x, abs, P.q_norm_w, P.eps, P.cos_lut, P.sin_lut, g, P.prologue);
+        if constexpr (FUSE) {
+            norm_rope_frag<HD>(x, abs, key ? P.k_norm_w : P.q_norm_w, P.eps, P.cos_lut, P.sin_lut, g, P.prologue,
+                               [&] { if constexpr (LATE) load_tile(kb, kA, vA, false); });
+            if (key) {
+                put_key(abs - pos0, x);
+#pragma unroll
+                for (int st = 0; st < NS; ++st)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[st][j] = 0.0f; /* no query */
+            }
+        }
 #pragma unroll
         for (int st = 0; st < NS; ++st)
 #pragma unroll
@@ -462,56 +546,31 @@ __device__ __forceinline__ void run_segment(const SplitParams &P, uint16_t *vt, 
     const uint32_t free_hi = min(pos0, ke - 1u);
 
 
-    /* ---- fused prologue: the rows of this call's positions -------------------
-     * Keys >= pos0 are the new tokens.  Before the key loop, the wave whose
-     * range [kb, ke) holds new keys builds those rows from the raw k/v
-     * (normalised, rotated, RNE fp16), stores them at their cache slots and
-     * stages them in its LDS area `fresh` ([n_rows][HD] K, then V).  Each new
-     * key lies in exactly one segment of the plan, so each row is stored once,
-     * and no other wave reads those bytes in this launch.  In the loop, the
-     * sub-tiles that reach pos0 take those rows from LDS in place of what was
-     * loaded from the slots (lanes clamped past ke take the last key's row
-     * too, so no stale slot content enters the product); the loop itself
-     * issues no extra global memory operations. */
-    const bool has_fresh = FUSE && ke > pos0;
     if constexpr (FUSE) {
         if (has_fresh) {
-            uint16_t *kw = const_cast<uint16_t *>(P.k_seq ? P.k_seq[s] : P.k_base + (size_t)s * P.seq_stride) +
-                           (size_t)kvh * HD;
-            uint16_t *vw = const_cast<uint16_t *>(P.v_seq ? P.v_seq[s] : P.v_base + (size_t)s * P.seq_stride) +
-                           (size_t)kvh * HD;
-            const uint32_t r0 = max(kb, pos0) - pos0, r1 = ke - pos0; /* rows of this segment */
-            for (uint32_t rb = r0; rb < r1; rb += 16u) {
-                const uint32_t r  = rb + (uint32_t)l16;
-                const bool real   = r < r1;
-                float x[NS][8];
-                if (real) {
-                    const float *kp = P.k_new + (((size_t)s * P.n_rows + r) * P.n_head_kv + kvh) * HD + 8 * g;
+            if (!spare)
+                for (uint32_t rb = r0; rb < r1; rb += 16u) {
+                    const uint32_t r = rb + (uint32_t)l16;
+                    const bool real  = r < r1;
+                    float x[NS][8];
+                    if (real) {
+                        const float *kp = P.k_new + (((size_t)s * P.n_rows + r) * P.n_head_kv + kvh) * HD + 8 * g;
 #pragma unroll
-                    for (int st = 0; st < NS; ++st) load8(kp + 32 * st, x[st]);
-                } else {
+                        for (int st = 0; st < NS; ++st) load8(kp + 32 * st, x[st]);
+                    } else {
 #pragma unroll
-                    for (int st = 0; st < NS; ++st)
+                        for (int st = 0; st < NS; ++st)
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) x[st][j] = 0.0f;
-                }
-                norm_rope_frag<HD>(x, real ? pos0 + r : pos0, P.k_norm_w, P.eps, P.cos_lut, P.sin_lut, g,
-                                   P.prologue);
-                if (real) {
-                    const size_t off = (size_t)lfm_slot_of(pos0 + r, P.window, P.cap) * row + 8 * g;
-#pragma unroll
-                    for (int st = 0; st < NS; ++st) {
-                        const u32x4_t w = pack8_rne(x[st]);
-                        *reinterpret_cast<u32x4_t *>(kw + off + 32 * st)                        = w;
-                        *reinterpret_cast<u32x4_t *>(fresh + (size_t)r * HD + 8 * g + 32 * st) = w;
+                            for (int j = 0; j < 8; ++j) x[st][j] = 0.0f;
                     }
+                    norm_rope_frag<HD>(x, real ? pos0 + r : pos0, P.k_norm_w, P.eps, P.cos_lut, P.sin_lut, g,
+                                       P.prologue, [] {});
+                    if (real) put_key(r, x);
                 }
-            }
             for (uint32_t e = r0 * CH + (uint32_t)lane; e < r1 * CH; e += 64u) {
                 const uint32_t r = e / CH, c = e % CH;
-                float x[8];
-                load8(P.v_new + (((size_t)s * P.n_rows + r) * P.n_head_kv + kvh) * HD + 8 * c, x);
-                const u32x4_t w = pack8_rne(x);
+                if (e >= r0 * CH + 64u) load8(P.v_new + (((size_t)s * P.n_rows + r) * P.n_head_kv + kvh) * HD + 8 * c, vraw);
+                const u32x4_t w = pack8_rne(vraw);
                 *reinterpret_cast<u32x4_t *>(vw + (size_t)lfm_slot_of(pos0 + r, P.window, P.cap) * row + 8 * c) = w;
                 *reinterpret_cast<u32x4_t *>(fresh + (size_t)(P.n_rows + r) * HD + 8 * c)                     = w;
             }

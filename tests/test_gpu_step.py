@@ -174,3 +174,46 @@ def test_step_matches_two_launch_path(gpu, orc):
     assert np.array_equal(outs[0], outs[1])
     for a, b in zip(*caches):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nq,nkv,hd,rows", [(15, 1, 64, 1),    # 15 query columns, the new key row in the last one
+                                            (16, 1, 64, 1),    # none left
+                                            (8, 2, 128, 3),    # 12 columns and 3 rows
+                                            (10, 2, 128, 3),   # 15 and 3: one tile, no room
+                                            (4, 4, 64, 8)])    # 8 and 8: exactly full
+@pytest.mark.parametrize("norms", ["both", "none", "q", "k"])
+@pytest.mark.parametrize("plan", ["grid", "balanced", "wg"])
+def test_step_key_rows_in_spare_columns(gpu, nq, nkv, hd, rows, norms, plan):
+    """New key rows that share the query tile's pass, fill it, or do not fit,
+    with either norm absent: caches equal to the prologue kernel's byte for
+    byte, outputs to the plain kernel's within fp32 sums (2^-22 relative per
+    probability, outputs below 4)."""
+    la = gpu
+    rng = np.random.default_rng(nq * hd + rows)
+    pos0 = np.array([0, 31, 100, 257], np.uint32)
+    n_seq, total = len(pos0), 257 + rows
+    cos, sin = (dev(la, t) for t in la.rope_lut_lfm3(total, hd, hd, 1e4, None))
+    qw, kw = (dev(la, (1 + 0.05 * rng.standard_normal(hd)).astype(np.float32)) for _ in range(2))
+    qw, kw = (qw if norms in ("both", "q") else None), (kw if norms in ("both", "k") else None)
+    k0 = [rand_kv(rng, int(p) + rows, nkv, hd) for p in pos0]
+    v0 = [rand_kv(rng, int(p) + rows, nkv, hd) for p in pos0]
+    q = rng.standard_normal((n_seq, rows, nq, hd), dtype=np.float32)
+    k = rng.standard_normal((n_seq, rows, nkv, hd), dtype=np.float32)
+    v = rng.standard_normal((n_seq, rows, nkv, hd), dtype=np.float32)
+    got = []
+    for fused in (True, False):
+        kd, vd = [dev(la, x) for x in k0], [dev(la, x) for x in v0]
+        kt, vt, pd, qd = la.pointer_table(kd), la.pointer_table(vd), dev(la, pos0), dev(la, q)
+        out = la.DeviceArray.zeros(q.shape, np.float32)
+        if fused:
+            with la.tuning(plan=plan):
+                la.gqa_f16_step(qd, dev(la, k), dev(la, v), None, True, kt, vt, pd, out, n_seq, rows, total, nq, nkv,
+                                hd, qw, kw, EPS, cos, sin)
+        else:
+            la.qkv_prologue(qd, dev(la, k), dev(la, v), kt, vt, pd, n_seq, rows, nq, nkv, hd, qw, kw, EPS, cos, sin)
+            la.gqa_f16_varlen(qd, None, True, kt, vt, pd, out, n_seq, rows, total, nq, nkv, hd)
+        got.append((out.numpy(), [x.numpy() for x in kd], [x.numpy() for x in vd]))
+    (o1, k1, v1), (o0, kp, vp) = got
+    for a, b in zip(k1 + v1, kp + vp):
+        assert np.array_equal(a, b)
+    assert np.abs(o1 - o0).max() <= 1e-5
