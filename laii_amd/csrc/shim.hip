@@ -100,6 +100,21 @@ static int noalloc_scratch(Scratch *out) {
 
 using lfm::AttnBatch;
 
+/* The engine context's step inputs (a few KB of pinned host memory): 16 bytes a
+ * lane over the host link, in one kernel launch. */
+static __global__ __launch_bounds__(256) void k_stage_in(uint4 *dst, const uint4 *src, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+extern "C" __attribute__((visibility("hidden"))) int lfm_ctx_stage_in(void *dst_dev, const void *src_pinned,
+                                                                      size_t bytes, lfm_attn_stream_t stream) {
+    const uint32_t n = (uint32_t)(bytes / 16u);
+    hipLaunchKernelGGL(k_stage_in, dim3((n + 255u) / 256u), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                       static_cast<uint4 *>(dst_dev), static_cast<const uint4 *>(src_pinned), n);
+    return lfm::hip_status(hipGetLastError());
+}
+
 static inline hipStream_t to_stream(lfm_attn_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0u; }
 static inline bool prologue_form_ok(int f) { return f == LFM_PROLOGUE_FAST || f == LFM_PROLOGUE_TABLE; }
