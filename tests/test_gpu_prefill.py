@@ -67,6 +67,32 @@ def test_prefill_cfg4_full_size_sampled(gpu, orc):
     assert np.allclose(got[:, 0], np.repeat(v0, 4, axis=1), atol=1e-6)
 
 
+@pytest.mark.parametrize("n_seq,n_tok,pos_0,nq,nkv", [
+    (1, 1, 0, 32, 8),      # 16 columns a wave; one key: the second group has none
+    (1, 1, 64, 8, 8),      # one key in the second group's first block
+    (2, 64, 0, 32, 2),     # kv_mul 16: tiles of four rows
+    (1, 65, 31, 16, 8),
+    (1, 704, 0, 32, 8),    # the last size at 16 columns (352 workgroups) ...
+    (1, 705, 0, 32, 8),    # ... and the first at 32
+    (1, 1100, 37, 32, 8),  # 32 columns, ragged
+    (1, 2300, 0, 32, 8),   # two groups at 64 columns
+    (1, 2049, 600, 16, 8),
+    (3, 1900, 3, 32, 8),   # one group
+])
+def test_prefill_tile_shapes(gpu, orc, n_seq, n_tok, pos_0, nq, nkv):
+    """Each tile width and group count of the launch, at the sizes where one
+    gives way to the next and at ragged ones: rows at the edges of 64-key blocks
+    and of the tiles against the oracle (same tolerance as every prefill)."""
+    rng = np.random.default_rng(n_tok + pos_0)
+    q, k16, v16, got = run_prefill(gpu, rng, n_seq, n_tok, pos_0, nq, nkv)
+    rows = sorted({r for e in (0, 16, 32, 64, 128, 640, n_tok) for r in (e - 1, e) if 0 <= r < n_tok})
+    for s in range(n_seq):
+        want = oracle_rows(orc, q, k16, v16, s, rows, pos_0, nq, nkv)
+        parity(got[s][rows], want, what=f"prefill tiles s={s} n={n_tok} pos0={pos_0}")
+    vmax = np.abs(f16_to_f32(v16)).max()
+    assert np.all(np.isfinite(got)) and np.abs(got).max() <= vmax + 1e-3
+
+
 def test_prefill_matches_decode_path(gpu):
     """The last prefill row equals the split-KV decode kernel at that position
     (two independent kernels, same cache)."""
