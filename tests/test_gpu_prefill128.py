@@ -101,6 +101,31 @@ def test_prefill128_window_vs_oracle(gpu, orc, n_tok, pos_0, window, kv_pos0):
         assert np.allclose(got, want, rtol=1e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("n_seq,n_tok,pos_0,window,kv_pos0,nq,nkv", [
+    (1, 63, 0, 0, 0, 16, 4),       # one group of waves
+    (1, 64, 0, 0, 0, 16, 4),       # two groups at 16 columns a wave
+    (1, 1, 63, 0, 0, 8, 8),        # one row
+    (1, 33, 31, 1, 31, 16, 4),     # tiles of one key block: the second group has none
+    (2, 130, 77, 0, 0, 32, 1),     # kv_mul 32: tiles of two rows
+    (1, 1001, 5, 256, 0, 16, 4),   # 252 workgroups, ragged
+    (1, 1040, 0, 256, 0, 16, 4),   # 260: one group
+    (1, 2049, 300, 0, 0, 16, 4),   # two groups at 32 columns
+    (3, 1370, 2, 0, 0, 16, 4),     # one group
+])
+def test_prefill128_tile_shapes(gpu, orc, n_seq, n_tok, pos_0, window, kv_pos0, nq, nkv):
+    """Each tile width and group count of the launch, at the sizes where one
+    gives way to the next: rows at the edges of 32-key blocks and of the tiles
+    against the oracle (same tolerance as every prefill)."""
+    rng = np.random.default_rng(n_tok + pos_0 + window)
+    q, k16, v16, g, got = run(gpu, rng, n_seq, n_tok, pos_0, nq, nkv, window=window, kv_pos0=kv_pos0)
+    rows = sorted({r for e in (0, 16, 32, 64, 256, 640, n_tok) for r in (e - 1, e) if 0 <= r < n_tok})
+    for s in range(n_seq):
+        want = oracle(orc, q, k16, v16, g, s, pos_0, kv_pos0, window, nq, nkv, rows=rows)
+        parity(got[s][rows], want, what=f"prefill128 tiles s={s} n={n_tok} pos0={pos_0} window={window}")
+    vmax = np.abs(f16_to_f32(v16)).max()
+    assert np.all(np.isfinite(got)) and np.abs(got).max() <= vmax + 1e-3
+
+
 def test_prefill128_lfm3_full_size_sampled(gpu, orc):
     """The bench workload (B 4 x 4096, 16q/4kv d128, gated full layer):
     sampled rows against the oracle, every output a gate-scaled convex
