@@ -103,12 +103,13 @@ def test_prefill128_window_vs_oracle(gpu, orc, n_tok, pos_0, window, kv_pos0):
 
 @pytest.mark.parametrize("n_seq,n_tok,pos_0,window,kv_pos0,nq,nkv", [
     (1, 63, 0, 0, 0, 16, 4),       # one group of waves
-    (1, 64, 0, 0, 0, 16, 4),       # two groups at 16 columns a wave
+    (1, 64, 0, 0, 0, 16, 4),       # two groups at 16 columns; the first tiles leave the second none
     (1, 1, 63, 0, 0, 8, 8),        # one row
-    (1, 33, 31, 1, 31, 16, 4),     # tiles of one key block: the second group has none
+    (1, 33, 31, 1, 31, 16, 4),     # a window: one group
     (2, 130, 77, 0, 0, 32, 1),     # kv_mul 32: tiles of two rows
-    (1, 1001, 5, 256, 0, 16, 4),   # 252 workgroups, ragged
-    (1, 1040, 0, 256, 0, 16, 4),   # 260: one group
+    (1, 1001, 5, 256, 0, 16, 4),   # a window, ragged
+    (2, 1024, 0, 0, 0, 16, 4),     # the last size at 16 columns (512 workgroups) ...
+    (2, 1025, 0, 0, 0, 16, 4),     # ... and one group after it
     (1, 2049, 300, 0, 0, 16, 4),   # two groups at 32 columns
     (3, 1370, 2, 0, 0, 16, 4),     # one group
 ])
