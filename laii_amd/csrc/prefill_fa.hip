@@ -85,17 +85,11 @@ __device__ __forceinline__ float4_t mfma(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-/* exp2 of two scores (log2 units) in fp32, packed to fp16, rounded to nearest
- * (RNE) or toward zero, a bias that leaves with the division by l.  Two groups
- * at 32 and 64 columns take RNE: 1.84e-4 from 64 bits against 2.25e-4 (1 x 1000
- * tokens).  16 columns keep the other, whose largest difference on isolated
- * huge scores is smaller, 1.82e-3 against 2.15e-3 (as one group: 2.03e-4 and
- * 2.03e-4 at 257 tokens). */
-template <bool RNE>
+/* exp2 of two scores (log2 units) in fp32, packed to fp16 with round
+ * toward zero */
 __device__ __forceinline__ half2_t exp_pk(float a, float b) {
-    const float ea = __builtin_amdgcn_exp2f(a), eb = __builtin_amdgcn_exp2f(b);
-    if constexpr (RNE) return half2_t{(_Float16)ea, (_Float16)eb};
-    else return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(ea, eb));
+    return __builtin_bit_cast(half2_t,
+                              __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_exp2f(a), __builtin_amdgcn_exp2f(b)));
 }
 
 /* transposing LDS read: within each 16-lane group, lane l receives element
@@ -342,10 +336,10 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
             const float4_t a = sc[0][nt], c = sc[1][nt];
             /* scalar temporaries: a bit_cast of an ext-vector element was
              * miscompiled into four reads of element 0 */
-            const half2_t h0 = exp_pk<(G > 1 && NT > 1)>(a[0], a[1]);
-            const half2_t h1 = exp_pk<(G > 1 && NT > 1)>(a[2], a[3]);
-            const half2_t h2 = exp_pk<(G > 1 && NT > 1)>(c[0], c[1]);
-            const half2_t h3 = exp_pk<(G > 1 && NT > 1)>(c[2], c[3]);
+            const half2_t h0 = exp_pk(a[0], a[1]);
+            const half2_t h1 = exp_pk(a[2], a[3]);
+            const half2_t h2 = exp_pk(c[0], c[1]);
+            const half2_t h3 = exp_pk(c[2], c[3]);
             u32x4_t w;
             w[0] = __builtin_bit_cast(uint32_t, h0);
             w[1] = __builtin_bit_cast(uint32_t, h1);
