@@ -7,11 +7,11 @@
  * attends keys [0, pos_0 + i] of its cache (causal by write order).  This
  * kernel computes all rows of a prompt in one launch.
  *
- * Workgroup = G groups of 4 waves; each group = TQ query positions x kv_mul
- * query heads of one KV head (64 NT query columns, TQ = 64 NT / kv_mul), so
- * each K/V block staged in LDS serves every query head that reads it.  With two
- * groups both hold the same columns and take the tile's key blocks in turn,
- * each with its own ring, and join O, m and l through LDS at the end.
+ * Workgroup = 4 waves = TQ query positions x kv_mul query heads of one KV
+ * head (64 NT query columns, TQ = 64 NT / kv_mul), so each K/V block staged in
+ * LDS serves every query head that reads it.  A column's keys are taken in
+ * order from key 0 by one wave, and its maximum is its own, so a row's bits
+ * depend neither on the tile's width nor on the rows beside it.
  *
  * Staging: 64-key K and V blocks (row-major, 128-B rows) move from global
  * memory straight into a ring of 4 LDS blocks (global_load_lds_dwordx4, no
@@ -116,17 +116,14 @@ __device__ __forceinline__ void fetch16_lds(uint32_t voff, const void *sbase, ui
     asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
 }
 
-template <int HD, int NT, int G>
-__global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
+template <int HD, int NT>
+__global__ __launch_bounds__(256, 2) void k_prefill(const PrefillParams P) {
     static_assert(HD == 64, "prefill kernel is specialised for head_dim 64");
     constexpr int NM = HD / 16;
-    /* per group a ring of NBUF blocks, each K (8 KB) then V (8 KB) */
-    constexpr uint32_t RINGB = NBUF * 2 * BLKB;
-    __shared__ __attribute__((aligned(1024))) uint8_t rings[G * RINGB];
+    /* ring of NBUF blocks, each K (8 KB) then V (8 KB) */
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[NBUF * 2 * BLKB];
 
-    const uint32_t gr = G > 1 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) : 0u;
-    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-    uint8_t *const ring = rings + gr * RINGB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
     /* 1-D grid, heaviest query tiles first across all (sequence, KV head)
      * pairs; consecutive workgroups take consecutive pairs, so with a pair
@@ -145,13 +142,10 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
     const uint32_t lo_pos = P.pos_0 + t0;                               /* smallest query position */
     const uint32_t hi_pos = P.pos_0 + min(t0 + P.tq, P.n_tok) - 1u;     /* largest query position  */
     const uint32_t n_keys = hi_pos + 1u;
-    /* this group's blocks gr, gr + G, ... of the tile, and its steps in them;
-     * steps [0, nfull) lie entirely at or below the lowest query row */
-    const uint32_t ablk  = (n_keys + KB - 1) / KB, asub = (n_keys + SB - 1) / SB;
-    const uint32_t afull = min((lo_pos + 1u) / SB, asub);
-    const uint32_t nblk  = (ablk + G - 1u - gr) / G;
-    const uint32_t nsub  = 2u * nblk - ((asub & 1u) && (ablk - 1u) % G == gr ? 1u : 0u);
-    const uint32_t nfull = 2u * (((afull >> 1) + G - 1u - gr) / G) + ((afull & 1u) && (afull >> 1) % G == gr ? 1u : 0u);
+    const uint32_t nblk   = (n_keys + KB - 1) / KB;
+    const uint32_t nsub   = (n_keys + SB - 1) / SB;
+    /* steps [0, nfull) lie entirely at or below the lowest query row */
+    const uint32_t nfull  = min((lo_pos + 1u) / SB, nsub);
 
     /* ---- staging: thread tid moves 16-B chunks tid and tid + 256 of each
      * 8-KB K and V block; chunk p sits at byte 16*p of the block (row p/8,
@@ -169,8 +163,8 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
     const uint32_t ring_lds = (uint32_t)(uintptr_t)ring; /* LDS address of the ring */
     const size_t blk_bytes  = (size_t)KB * row * sizeof(uint16_t);
     /* 4 fetches per wave and block (vmcnt counts them) */
-    auto fetch_block = [&](uint32_t b) {
-        const uint32_t slot = ring_lds + (b % NBUF) * (2 * BLKB), blk = b * G + gr;
+    auto fetch_block = [&](uint32_t blk) {
+        const uint32_t slot = ring_lds + (blk % NBUF) * (2 * BLKB);
         if ((blk + 1u) * KB <= n_keys) {
             /* a whole block: uniform base, fixed per-lane offsets */
             const uint8_t *kb = reinterpret_cast<const uint8_t *>(kc) + blk * blk_bytes;
@@ -197,7 +191,7 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
     /* the first two blocks are in flight before the Q loads: the wait for Q
      * (which also covers these older fetches) then takes one memory round
      * trip, not two */
-    if (G == 1 || nblk > 0u) fetch_block(0u);
+    fetch_block(0u);
     if (nblk > 1u) fetch_block(1u);
 
     /* ---- columns of this lane: (head j, row t) per N-tile -------------- */
@@ -282,7 +276,7 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
                 for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const uint32_t key = ((k >> 1) * G + gr) * KB + (k & 1u) * SB + (uint32_t)(16 * mt + 4 * g + i);
+                        const uint32_t key = k * SB + (uint32_t)(16 * mt + 4 * g + i);
                         if (key > col_pos[nt]) sc[mt][nt][i] = -INFINITY;
                     }
         }
@@ -374,11 +368,11 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
     };
 
     /* ---- steps: P(k) and PV(k), then S^T(k + 1) in the same registers -- */
+    enter_block(0u);
     float4_t scur[2][NT];
-    if (G == 1 || nblk > 0u) {
-        enter_block(0u);
-        if (nfull > 0u) scores(std::false_type{}, 0u, scur);
-        else scores(std::true_type{}, 0u, scur);
+    if (nfull > 0u) scores(std::false_type{}, 0u, scur);
+    else scores(std::true_type{}, 0u, scur);
+    {
         float mx[NT];
         const bool any_raise = step_max(std::true_type{}, scur, mx);
         rescale(std::true_type{}, any_raise, scur, mx);
@@ -425,54 +419,9 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
             ++k;
         }
     };
-    if (G == 1 || nblk > 0u) {
-        run_steps(std::false_type{}, nfull > 0u ? nfull - 1u : 0u); /* S^T(k + 1) unmasked */
-        run_steps(std::true_type{}, nsub - 1u);
-        accumulate(k, scur);
-    }
-
-    /* ---- two groups: each hands half of O (with its m and l) to the other
-     * through its own ring and finishes the other half.  A group without keys
-     * at or below a column's row has l = 0 there and counts for nothing. */
-    if constexpr (G == 2) {
-        constexpr int NH = NM / 2;
-        /* one barrier per block of group 0, which has as many or one more; then
-         * every wave is past its last read of the rings */
-        if (nblk < (ablk + 1u) / 2u) __syncthreads();
-        __syncthreads();
-        float4_t *xo = reinterpret_cast<float4_t *>(ring);
-        float2 *xm   = reinterpret_cast<float2 *>(ring + NT * NH * 4096);
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            xm[nt * 256 + tid] = make_float2(negm[nt][0], lacc[nt][0]);
-#pragma unroll
-            for (int mh = 0; mh < NH; ++mh) xo[(nt * NH + mh) * 256 + tid] = gr ? oacc[mh][nt] : oacc[NH + mh][nt];
-        }
-        __syncthreads();
-        const uint8_t *other = rings + (1u - gr) * RINGB;
-        const float4_t *yo   = reinterpret_cast<const float4_t *>(other);
-        const float2 *ym     = reinterpret_cast<const float2 *>(other + NT * NH * 4096);
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const float2 o = ym[nt * 256 + tid];
-            const float l0 = lacc[nt][0], m0 = l0 == 0.0f ? -INFINITY : -negm[nt][0];
-            const float m1 = o.y == 0.0f ? -INFINITY : -o.x, m = fmaxf(m0, m1);
-            const float f0 = l0 == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m0 - m);
-            const float f1 = o.y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
-            const float lt = l0 * f0 + o.y * f1, inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-            if (!col_ok[nt]) continue;
-            const uint32_t c = (uint32_t)(wave * (16 * NT) + nt * 16 + l16);
-            const uint32_t j = c / P.tq, t = t0 + c % P.tq;
-            float *op = P.out + (((size_t)s * P.n_tok + t) * P.n_head_q + kvh * P.kv_mul + j) * HD + gr * (16 * NH) + 4 * g;
-#pragma unroll
-            for (int mh = 0; mh < NH; ++mh) {
-                const float4_t a = gr ? oacc[NH + mh][nt] : oacc[mh][nt], b = yo[(nt * NH + mh) * 256 + tid];
-                const float4_t x = (a * f0 + b * f1) * inv;
-                *reinterpret_cast<float4 *>(op + 16 * mh) = make_float4(x[0], x[1], x[2], x[3]);
-            }
-        }
-        return;
-    }
+    run_steps(std::false_type{}, nfull > 0u ? nfull - 1u : 0u); /* S^T(k + 1) unmasked */
+    run_steps(std::true_type{}, nsub - 1u);
+    accumulate(k, scur);
 
     /* ---- epilogue: O / l ------------------------------------------------- */
 #pragma unroll
@@ -491,49 +440,41 @@ __global__ __launch_bounds__(256 * G, 2) void k_prefill(const PrefillParams P) {
     }
 }
 
-struct PrefillShape {
-    uint32_t nt, groups, n_wg;
-};
-
 } // namespace
 
 bool prefill_supports(uint32_t head_dim, uint32_t kv_mul) {
     return head_dim == 64u && kv_mul >= 1u && kv_mul <= 16u && (256u % kv_mul) == 0u;
 }
 
-/* Columns per wave (16 nt) and key groups.  nt = 4 with one group has the
- * least work per score, but its workgroups are few and long: 1 x 2000 tokens of
- * 32q/8kv are 256 of them, one a CU, and the longest alone takes 41.8 us.
- * Narrower tiles make more workgroups, and two groups halve their chain of
- * steps.  Measured on MI355X, us (nt, groups: 4,1 / 4,2 / 2,2 / 1,2), 32q/8kv:
- *   sequences x tokens     4,1    4,2    2,2    1,2
- *        1 x  256         10.8   13.0    8.0    5.8
- *        1 x  512         15.6   16.6   10.2    7.8
- *        1 x  700         18.8   19.1   12.1   10.7   352 workgroups at nt 1
- *        2 x  384         13.7   15.5    9.6    9.8   384
- *        1 x 1000         23.7   22.9   14.9   15.1   500
- *        1 x 2000         41.8   37.0   29.0   38.2   504 at nt 2
- *        4 x  512         17.6   18.9   16.8   21.4   512
- *        1 x 2500         54.1   44.4   45.3   55.0   632; 320 at nt 4
- *        1 x 4096         95.4   81.5   90.6  121.1   512 at nt 4
- *        2 x 2000         51.1   50.3   55.3   74.2   512
- *        4 x 1000         31.2   36.3   39.9   51.9   512
- *        2 x 2500         66.9   76.9   78.9  105.9   640
- * The lightest tiles run last, so a little over one round of workgroups (a CU
- * holds one of two groups) still ends early; two groups at nt 4 pay where
- * the longest tile has 64 steps or more. */
-static PrefillShape prefill_shape(uint32_t n_seq, uint32_t n_tok, uint32_t n_head_q, uint32_t n_head_kv) {
-    const uint32_t mul = n_head_q / n_head_kv;
-    auto wgs = [&](uint32_t nt) {
-        const uint32_t tq = 64u * nt / mul;
-        return (uint64_t)((n_tok + tq - 1u) / tq) * n_head_kv * n_seq;
+/* Columns per wave, in tiles of 16.  Four have the least work per score, but
+ * their workgroups are few and long: 1 x 2000 tokens of 32q/8kv are 256 of them,
+ * one a CU, and the longest alone takes 41.9 us.  Narrower tiles make more and
+ * shorter ones, with the same bits.  A CU holds two workgroups, so the launch takes
+ * about as long as its longest tile (pos_0 + n_tok keys) while the steps of all
+ * (pos_0 + n_tok / 2 keys on average) make no more than that in each of 512
+ * slots; past that line the wider form is taken.  Measured on MI355X, us, 32q/8kv:
+ *   sequences x tokens     4 tiles  2 tiles  1 tile   workgroups
+ *        1 x  256           10.8      7.3      5.7
+ *        1 x 1000           23.6     17.0     14.1
+ *        1 x 2000           41.9     32.6     29.5    1000 at 1 tile
+ *        2 x 1000           24.9     19.8     19.3    1008
+ *        4 x  512           17.7     13.6     14.3    1024
+ *        3 x  700           21.8     16.0     17.5    1056
+ *        1 x 2500           53.8     40.8     45.0    1256
+ *        2 x  700 at 1400   44.0     35.3     41.4     704; mean tile 0.83 of the longest
+ *        1 x 1000 at 1000   40.5     29.5     24.8     504
+ *        2 x 2000           50.6     44.4     55.9    1008 at 2 tiles
+ *        1 x 4096           94.9     79.6    101.6    1024
+ *        3 x 1500           41.8     42.3     50.8    1128
+ *        2 x 2500           65.8     66.9     81.5    1264 */
+static uint32_t prefill_tiles(uint32_t n_seq, uint32_t n_tok, uint32_t pos_0, uint32_t n_head_kv, uint32_t kv_mul) {
+    const uint64_t longest = (uint64_t)pos_0 + n_tok, twice_mean = 2u * (uint64_t)pos_0 + n_tok;
+    auto steps = [&](uint32_t nt) { /* of all workgroups, in longest tiles per 1024 */
+        const uint32_t tq = 64u * nt / kv_mul;
+        return (uint64_t)((n_tok + tq - 1u) / tq) * n_head_kv * n_seq * twice_mean;
     };
-    PrefillShape sh{4u, 1u, 0u};
-    if (wgs(1u) <= 352u) sh = {1u, 2u, 0u};
-    else if (wgs(2u) <= 512u) sh = {2u, 2u, 0u};
-    else if (wgs(4u) <= 512u && n_tok >= 2048u) sh = {4u, 2u, 0u};
-    sh.n_wg = (uint32_t)wgs(sh.nt);
-    return sh;
+    if (steps(1u) < 1024u * longest) return 1u;
+    return steps(2u) <= 1024u * longest ? 2u : 4u;
 }
 
 int launch_prefill(const float *q, const uint16_t *k, const uint16_t *v, float *out,
@@ -556,14 +497,13 @@ int launch_prefill(const float *q, const uint16_t *k, const uint16_t *v, float *
     hipEvent_t ev0, ev1;
     profile_events(&ev0, &ev1);
     if (ev0) (void)hipEventRecord(ev0, stream);
-    const PrefillShape sh = prefill_shape(n_seq, n_tok, n_head_q, n_head_kv);
-    P.tq       = 64u * sh.nt / P.kv_mul;
+    const uint32_t nt = prefill_tiles(n_seq, n_tok, pos_0, n_head_kv, P.kv_mul);
+    P.tq       = 64u * nt / P.kv_mul;
     P.n_qtiles = (n_tok + P.tq - 1u) / P.tq;
-    const dim3 grid(sh.n_wg), block(256u * sh.groups);
-    if (sh.nt == 1u) hipLaunchKernelGGL((k_prefill<64, 1, 2>), grid, block, 0, stream, P);
-    else if (sh.nt == 2u) hipLaunchKernelGGL((k_prefill<64, 2, 2>), grid, block, 0, stream, P);
-    else if (sh.groups == 2u) hipLaunchKernelGGL((k_prefill<64, 4, 2>), grid, block, 0, stream, P);
-    else hipLaunchKernelGGL((k_prefill<64, 4, 1>), grid, block, 0, stream, P);
+    const dim3 grid(P.n_qtiles * n_head_kv * n_seq);
+    if (nt == 1u) hipLaunchKernelGGL((k_prefill<64, 1>), grid, dim3(256), 0, stream, P);
+    else if (nt == 2u) hipLaunchKernelGGL((k_prefill<64, 2>), grid, dim3(256), 0, stream, P);
+    else hipLaunchKernelGGL((k_prefill<64, 4>), grid, dim3(256), 0, stream, P);
     hipError_t e = hipGetLastError();
     if (ev1) (void)hipEventRecord(ev1, stream);
     (void)head_dim;

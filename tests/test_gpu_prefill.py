@@ -68,21 +68,21 @@ def test_prefill_cfg4_full_size_sampled(gpu, orc):
 
 
 @pytest.mark.parametrize("n_seq,n_tok,pos_0,nq,nkv", [
-    (1, 1, 0, 32, 8),      # 16 columns a wave; one key: the second group has none
-    (1, 1, 64, 8, 8),      # one key in the second group's first block
+    (1, 1, 0, 32, 8),      # 16 columns a wave; one key
+    (1, 1, 64, 8, 8),      # one key in the second block
     (2, 64, 0, 32, 2),     # kv_mul 16: tiles of four rows
     (1, 65, 31, 16, 8),
-    (1, 704, 0, 32, 8),    # the last size at 16 columns (352 workgroups) ...
-    (1, 705, 0, 32, 8),    # ... and the first at 32
-    (1, 1100, 37, 32, 8),  # 32 columns, ragged
-    (1, 2300, 0, 32, 8),   # two groups at 64 columns
+    (1, 704, 0, 32, 8),
+    (1, 705, 0, 32, 8),
+    (1, 1100, 37, 32, 8),  # ragged
+    (1, 2300, 0, 32, 8),   # 32 columns
     (1, 2049, 600, 16, 8),
-    (3, 1900, 3, 32, 8),   # one group
+    (3, 1900, 3, 32, 8),   # 64 columns
 ])
 def test_prefill_tile_shapes(gpu, orc, n_seq, n_tok, pos_0, nq, nkv):
-    """Each tile width and group count of the launch, at the sizes where one
-    gives way to the next and at ragged ones: rows at the edges of 64-key blocks
-    and of the tiles against the oracle (same tolerance as every prefill)."""
+    """Each tile width of the launch, at ragged sizes: rows at the edges of
+    64-key blocks and of the tiles against the oracle (same tolerance as every
+    prefill)."""
     rng = np.random.default_rng(n_tok + pos_0)
     q, k16, v16, got = run_prefill(gpu, rng, n_seq, n_tok, pos_0, nq, nkv)
     rows = sorted({r for e in (0, 16, 32, 64, 128, 640, n_tok) for r in (e - 1, e) if 0 <= r < n_tok})
@@ -91,6 +91,54 @@ def test_prefill_tile_shapes(gpu, orc, n_seq, n_tok, pos_0, nq, nkv):
         parity(got[s][rows], want, what=f"prefill tiles s={s} n={n_tok} pos0={pos_0}")
     vmax = np.abs(f16_to_f32(v16)).max()
     assert np.all(np.isfinite(got)) and np.abs(got).max() <= vmax + 1e-3
+
+
+def patterned(rng, pattern, n_tok, nq, nkv, hd=64):
+    """q, k, v of one prompt: N(0,1) data, or keys that share a direction with
+    every query, with scores that climb along the sequence ("rising"), are huge
+    on single keys ("spike"), large at first ("falling"), or below -128 log2
+    units at first ("sunk")."""
+    q = rng.standard_normal((1, n_tok, nq, hd), dtype=np.float32)
+    k = rng.standard_normal((1, n_tok, nkv, hd), dtype=np.float32) * np.float32(0.5)
+    v = f16(rng.standard_normal((1, n_tok, nkv, hd), dtype=np.float32))
+    if pattern != "plain":
+        u = rng.standard_normal(hd).astype(np.float32)
+        u /= np.linalg.norm(u)
+        q += 3.0 * u
+        t = np.arange(n_tok, dtype=np.float32)
+        amp = {"rising": 0.25 * t, "spike": np.where(t % 97 == 40, 60.0, 0.0),
+               "falling": np.where(t < 64, 40.0, 0.0), "sunk": np.where(t < 32, -400.0, 0.0)}[pattern]
+        k += amp.astype(np.float32)[None, :, None, None] * u
+    return q, f16(k), v
+
+
+@pytest.mark.parametrize("pattern", ["plain", "rising", "spike", "falling", "sunk"])
+@pytest.mark.parametrize("nq,nkv,some,many", [(32, 8, 4, 8), (8, 8, 13, 26), (16, 8, 7, 13), (32, 4, 4, 8)])
+def test_prefill_row_bits_do_not_depend_on_the_call(gpu, orc, pattern, nq, nkv, some, many):
+    """A prompt alone (16 columns a wave), among `some` sequences (32) and among
+    `many` (64), whole and in two pieces: every row the same bits, and the
+    rows of the first call within tolerance of the oracle."""
+    la = gpu
+    rng = np.random.default_rng(nq * 10 + nkv)
+    n_tok, cut, hd = 600, 250, 64
+    q, k16, v16 = patterned(rng, pattern, n_tok, nq, nkv)
+
+    def call(n_seq, lo, hi):
+        rep = lambda x, n: np.broadcast_to(x[:, :n], (n_seq, n, *x.shape[2:]))  # noqa: E731
+        out = la.DeviceArray.zeros((n_seq, hi - lo, nq, hd), np.float32)
+        la.prefill_f16(dev(la, np.broadcast_to(q[:, lo:hi], (n_seq, hi - lo, nq, hd))), dev(la, rep(k16, hi)),
+                       dev(la, rep(v16, hi)), out, n_seq, hi - lo, lo, hi * nkv * hd, nq, nkv, hd)
+        return out.numpy().view(np.uint32)
+
+    one = call(1, 0, n_tok)[0]
+    rows = [0, 1, 15, 31, 32, 63, 64, 65, 127, 128, 249, 250, 300, 511, 512, 599]
+    got = one.view(np.float32)[rows]
+    parity(got, oracle_rows(orc, q, k16, v16, 0, rows, 0, nq, nkv), what=f"prefill {pattern} {nq}q/{nkv}kv")
+    for n_seq in (some, many):
+        assert np.all(call(n_seq, 0, n_tok) == one), f"{n_seq} sequences"
+    for n_seq in (1, some, many):
+        assert np.all(call(n_seq, 0, cut) == one[:cut]), f"{n_seq} sequences, first piece"
+        assert np.all(call(n_seq, cut, n_tok) == one[cut:]), f"{n_seq} sequences, second piece"
 
 
 def test_prefill_matches_decode_path(gpu):
