@@ -93,10 +93,8 @@ int lfm_attn_plan_preview(uint32_t n_seq, uint32_t n_rows, uint32_t n_head_q, ui
  * position pos_0, sliding window or 0, head shape) under the current
  * overrides: out4 = {query positions per tile, tiles per workgroup, short
  * tiles at the sequence start dispatched first (their window reaches before
- * position 0), workgroups}.  This is the shape with one group of waves per
- * tile; a head_dim-128 full-layer launch of few workgroups divides it (two groups
- * share a tile's keys, on tiles as wide or half as wide, longest first).
- * LFM_ATTN_E_UNSUPPORTED for a head shape that entry point does not take. */
+ * position 0), workgroups}.  LFM_ATTN_E_UNSUPPORTED for a head shape that
+ * entry point does not take. */
 int lfm_attn_prefill_plan_preview(uint32_t n_seq, uint32_t n_tok, uint32_t pos_0, uint32_t window_len,
                                   uint32_t n_head_q, uint32_t n_head_kv, uint32_t head_dim, uint32_t out4[4]);
 

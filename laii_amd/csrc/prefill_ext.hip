@@ -13,11 +13,9 @@
  * (kv_pos0 = 0) and a sliding-window layer a linear staging copy of the
  * window before the prompt plus the prompt's rows.
  *
- * Workgroup = G groups of 4 waves; each group = 64 NT query columns: TQ = 64
- * NT / kv_mul positions x kv_mul query heads of one KV head, so each K/V block
- * staged in LDS serves every query head that reads it; 16 NT columns per wave.
- * With two groups both hold the same columns and take one half of the tile's
- * key blocks each, with its own ring, and join O, m and l through LDS.
+ * Workgroup = 4 waves = 128 query columns: TQ = 128 / kv_mul positions x
+ * kv_mul query heads of one KV head, so each K/V block staged in LDS serves
+ * every query head that reads it; 32 columns per wave.
  *
  * Each 32-key block of K (and of V) is kept in LDS as two 64-dim halves of
  * [32 keys][128 B], with the 16-B chunks of row r XOR-swizzled by
@@ -66,6 +64,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int KB       = 32;            /* keys per block (one compute step)       */
 constexpr int NBUF     = 4;             /* LDS ring of blocks                      */
 constexpr int HALFB    = KB * 128;      /* bytes of one 64-dim half of a block     */
+constexpr int NT       = 2;             /* 16-column tiles per wave                */
 constexpr float kLazy  = 8.0f;          /* headroom in log2 units (P <= 2^8)        */
 
 struct PrefillExtParams {
@@ -89,14 +88,9 @@ __device__ __forceinline__ float4_t mfma(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-/* exp2 of two scores (log2 units) in fp32, packed to fp16, rounded to nearest
- * (RNE, with two groups: 1.83e-4 from 64 bits against 2.27e-4 at 1 x 1000
- * tokens) or toward zero, a bias that leaves with the division by l */
-template <bool RNE>
 __device__ __forceinline__ half2_t exp_pk(float a, float b) {
-    const float ea = __builtin_amdgcn_exp2f(a), eb = __builtin_amdgcn_exp2f(b);
-    if constexpr (RNE) return half2_t{(_Float16)ea, (_Float16)eb};
-    else return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(ea, eb));
+    return __builtin_bit_cast(half2_t,
+                              __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_exp2f(a), __builtin_amdgcn_exp2f(b)));
 }
 
 /* transposing LDS read: within each 16-lane group, lane l receives element
@@ -129,7 +123,7 @@ struct TileGeom {
     uint32_t t0, lo_pos, hi_pos, r_hi, b_lo, b_hi, u0, u1;
 };
 
-__device__ __forceinline__ TileGeom tile_geom(const PrefillExtParams &P, uint32_t qt, uint32_t groups, uint32_t gr) {
+__device__ __forceinline__ TileGeom tile_geom(const PrefillExtParams &P, uint32_t qt) {
     TileGeom t;
     t.t0     = qt * P.tq;
     t.lo_pos = P.pos_0 + t.t0;
@@ -142,11 +136,6 @@ __device__ __forceinline__ TileGeom tile_geom(const PrefillExtParams &P, uint32_
     const uint32_t free_key_lo = P.window && t.hi_pos + 1u > P.window ? t.hi_pos + 1u - P.window : 0u;
     const uint32_t b_free = free_key_lo > P.kv_pos0 ? (free_key_lo - P.kv_pos0 + KB - 1u) / KB : 0u;
     const uint32_t b_diag = (t.lo_pos - P.kv_pos0 + 1u) / KB;
-    if (groups == 2u) { /* this group's half of the blocks: the first has as many or one more */
-        const uint32_t mid = t.b_lo + (t.b_hi - t.b_lo + 1u) / 2u;
-        if (gr) t.b_lo = mid;
-        else t.b_hi = mid;
-    }
     t.u0 = min(max(t.b_lo, b_free), t.b_hi);
     t.u1 = max(t.u0, min(t.b_hi, b_diag));
     return t;
@@ -159,18 +148,15 @@ __device__ __forceinline__ TileGeom tile_geom(const PrefillExtParams &P, uint32_
  * in flight while the current tile finishes, and a sliding-window tile --
  * about window / 32 blocks -- does not pay the workgroup's set-up and the
  * ring's fill on its own. */
-template <int HD, int NT, int G>
-__global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill_ext(const PrefillExtParams P) {
+template <int HD>
+__global__ __launch_bounds__(256, HD == 64 ? 3 : 2) void k_prefill_ext(const PrefillExtParams P) {
     constexpr int NH   = HD / 64;            /* 64-dim halves per row              */
     constexpr int BLKB = 2 * NH * HALFB;     /* K halves, then V halves            */
     constexpr int NS   = HD / 32;            /* k-steps of Q.K^T                   */
     constexpr int NM   = HD / 16;            /* 16-dim tiles of O^T                */
-    constexpr int RINGB = NBUF * BLKB;       /* one ring per group                 */
-    __shared__ __attribute__((aligned(1024))) uint8_t rings[G * RINGB];
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[NBUF * BLKB];
 
-    const uint32_t gr = G > 1 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) : 0u;
-    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-    uint8_t *const ring = rings + gr * RINGB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, g = lane >> 4;
     /* 1-D grid, heaviest chains first; consecutive workgroups take
      * consecutive (sequence, KV head) pairs.  With n_light > 0 (one tile per
@@ -213,11 +199,11 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
      * block being entered */
     uint32_t n_stream = 0;
     for (uint32_t qt = qt_first; qt < qt_end; ++qt) {
-        const TileGeom t = tile_geom(P, qt, G, gr);
+        const TileGeom t = tile_geom(P, qt);
         n_stream += t.b_hi - t.b_lo;
     }
     uint32_t f_qt = qt_first, f_j = 0;
-    TileGeom fg   = tile_geom(P, f_qt, G, gr);
+    TileGeom fg   = tile_geom(P, f_qt);
     uint32_t f_b  = fg.b_lo;
     /* 2 NH fetches per wave and block (vmcnt counts them) */
     auto fetch_next = [&]() {
@@ -246,7 +232,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
         }
         ++f_j;
         if (++f_b == fg.b_hi && ++f_qt < qt_end) {
-            fg  = tile_geom(P, f_qt, G, gr);
+            fg  = tile_geom(P, f_qt);
             f_b = fg.b_lo;
         }
     };
@@ -254,7 +240,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
     /* the first two blocks are in flight before the first tile's Q loads:
      * the wait for Q (which also covers these older fetches) then takes one
      * memory round trip, not two */
-    if (G == 1 || n_stream > 0u) fetch_next();
+    fetch_next();
     if (n_stream > 1u) fetch_next();
 
     /* fragment offsets within a 64-dim half (bytes).  K: row 16*mt + l16,
@@ -283,7 +269,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
         const uint32_t t0_ = qt_ * P.tq;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const uint32_t c = (uint32_t)(wave * (16 * NT) + nt * 16 + l16);
+            const uint32_t c = (uint32_t)(wave * 32 + nt * 16 + l16);
             const uint32_t j = c / P.tq, t = t0_ + c % P.tq;
             const bool ok    = t < P.n_tok;
             gnext[nt] = (P.gate && ok) ? P.gate[((size_t)s * P.n_tok + t) * P.n_head_q + kvh * P.kv_mul + j] : 1.0f;
@@ -300,7 +286,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
 
     uint32_t j0 = 0; /* stream index of the current tile's first block */
     for (uint32_t qt = qt_first; qt < qt_end; ++qt) {
-        const TileGeom tg = tile_geom(P, qt, G, gr);
+        const TileGeom tg = tile_geom(P, qt);
         const uint32_t t0 = tg.t0;
         auto block_masked = [&](uint32_t b) { return b < tg.u0 || b >= tg.u1; };
         auto block_lds    = [&](uint32_t b) { return ring + ((j0 + b - tg.b_lo) % NBUF) * BLKB; };
@@ -312,7 +298,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
         float graw[NT]; /* the output gates (loaded with Q): the epilogue does not wait for them */
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const uint32_t c = (uint32_t)(wave * (16 * NT) + nt * 16 + l16);
+            const uint32_t c = (uint32_t)(wave * 32 + nt * 16 + l16);
             const uint32_t t = t0 + c % P.tq;
             col_ok[nt]  = t < P.n_tok;
             graw[nt]    = gnext[nt];
@@ -423,10 +409,10 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 const float4_t a = sc[0][nt], c = sc[1][nt];
-                const half2_t h0 = exp_pk<(G > 1)>(a[0], a[1]);
-                const half2_t h1 = exp_pk<(G > 1)>(a[2], a[3]);
-                const half2_t h2 = exp_pk<(G > 1)>(c[0], c[1]);
-                const half2_t h3 = exp_pk<(G > 1)>(c[2], c[3]);
+                const half2_t h0 = exp_pk(a[0], a[1]);
+                const half2_t h1 = exp_pk(a[2], a[3]);
+                const half2_t h2 = exp_pk(c[0], c[1]);
+                const half2_t h3 = exp_pk(c[2], c[3]);
                 u32x4_t w;
                 w[0] = __builtin_bit_cast(uint32_t, h0);
                 w[1] = __builtin_bit_cast(uint32_t, h1);
@@ -468,14 +454,11 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
         };
 
         const uint32_t b_lo = tg.b_lo, b_hi = tg.b_hi, u0 = tg.u0, u1 = tg.u1;
-        const bool some = G == 1 || b_hi > b_lo; /* a lone block leaves the second group none */
+        enter_block(b_lo);
         float4_t scur[2][NT];
-        if (some) {
-            enter_block(b_lo);
-            if (block_masked(b_lo)) scores(std::true_type{}, b_lo, scur);
-            else scores(std::false_type{}, b_lo, scur);
-            update_max(scur);
-        }
+        if (block_masked(b_lo)) scores(std::true_type{}, b_lo, scur);
+        else scores(std::false_type{}, b_lo, scur);
+        update_max(scur);
         /* step b: S^T(b + 1) into the other register set, then P(b) and PV(b);
          * two steps per iteration with the sets swapping roles */
         float4_t snxt[2][NT];
@@ -504,11 +487,9 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
         };
         /* blocks [u0, u1) need no mask; masked ones sit below (window edge)
          * and above (diagonal) */
-        if (some) {
-            run_steps(std::true_type{}, u0 > 0u ? u0 - 1u : 0u);
-            run_steps(std::false_type{}, u1 > 0u ? u1 - 1u : 0u);
-            run_steps(std::true_type{}, b_hi - 1u);
-        }
+        run_steps(std::true_type{}, u0 > 0u ? u0 - 1u : 0u);
+        run_steps(std::false_type{}, u1 > 0u ? u1 - 1u : 0u);
+        run_steps(std::true_type{}, b_hi - 1u);
         /* the next tile's Q loads before the last P.V; on the chain's last
          * tile the Q registers are cleared instead, so that no path carries
          * the loaded values through a whole tile (a conditional load alone
@@ -523,54 +504,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
                 for (int st = 0; st < NS; ++st) qraw[nt][st][0] = qraw[nt][st][1] = make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
-        if (some) accumulate(b, scur);
-        /* ---- two groups (one tile a workgroup): each hands half of O, with its
-         * m and l, to the other through its own ring and finishes the other
-         * half.  A group without keys of a column has l = 0 there and counts
-         * for nothing. */
-        if constexpr (G == 2) {
-            constexpr int NO = NM / 2;
-            /* one barrier per block of group 0, which has as many or one more;
-             * then every wave is past its last read of the rings */
-            const uint32_t all = tile_geom(P, qt, 1u, 0u).b_hi - tile_geom(P, qt, 1u, 0u).b_lo;
-            if (b_hi - b_lo < (all + 1u) / 2u) __syncthreads();
-            __syncthreads();
-            float4_t *xo = reinterpret_cast<float4_t *>(ring);
-            float2 *xm   = reinterpret_cast<float2 *>(ring + NT * NO * 4096);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                xm[nt * 256 + tid] = make_float2(negm[nt][0], lacc[nt][0]);
-#pragma unroll
-                for (int mo = 0; mo < NO; ++mo) xo[(nt * NO + mo) * 256 + tid] = gr ? oacc[mo][nt] : oacc[NO + mo][nt];
-            }
-            __syncthreads();
-            const uint8_t *other = rings + (1u - gr) * RINGB;
-            const float4_t *yo   = reinterpret_cast<const float4_t *>(other);
-            const float2 *ym     = reinterpret_cast<const float2 *>(other + NT * NO * 4096);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const float2 o = ym[nt * 256 + tid];
-                const float l0 = lacc[nt][0], m0 = l0 == 0.0f ? -INFINITY : -negm[nt][0];
-                const float m1 = o.y == 0.0f ? -INFINITY : -o.x, m = fmaxf(m0, m1);
-                const float f0 = l0 == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m0 - m);
-                const float f1 = o.y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
-                const float lt = l0 * f0 + o.y * f1;
-                float gv       = 1.0f;
-                if (P.gate) gv = P.gate_is_logit ? 1.0f / (1.0f + expf(-graw[nt])) : graw[nt];
-                const float inv = lt > 0.0f ? gv / lt : 0.0f;
-                if (!col_ok[nt]) continue;
-                const uint32_t c = (uint32_t)(wave * (16 * NT) + nt * 16 + l16);
-                const uint32_t j = c / P.tq, t = t0 + c % P.tq;
-                float *op = P.out + (((size_t)s * P.n_tok + t) * P.n_head_q + kvh * P.kv_mul + j) * HD + gr * (16 * NO) + 4 * g;
-#pragma unroll
-                for (int mo = 0; mo < NO; ++mo) {
-                    const float4_t a = gr ? oacc[NO + mo][nt] : oacc[mo][nt], y = yo[(nt * NO + mo) * 256 + tid];
-                    const float4_t x = (a * f0 + y * f1) * inv;
-                    *reinterpret_cast<float4 *>(op + 16 * mo) = make_float4(x[0], x[1], x[2], x[3]);
-                }
-            }
-            return;
-        }
+        accumulate(b, scur);
         /* ---- epilogue: O * gate / l ------------------------------------------ */
         float inv[NT];
 #pragma unroll
@@ -583,7 +517,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
             }
             inv[nt] = lt > 0.0f ? gv / lt : 0.0f;
         }
-        if (HD == 128 && NT == 2 && qt + 1u >= qt_end) {
+        if (HD == 128 && qt + 1u >= qt_end) {
             /* (head_dim 128: the head_dim-64 instance, at three waves per SIMD,
              * has no registers to spare for it.)
              * The workgroup's last tile: the ring is free once every wave's
@@ -625,7 +559,7 @@ __global__ __launch_bounds__(256 * G, HD == 64 && G == 1 ? 3 : 2) void k_prefill
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             if (!col_ok[nt]) continue;
-            const uint32_t c  = (uint32_t)(wave * (16 * NT) + nt * 16 + l16);
+            const uint32_t c  = (uint32_t)(wave * 32 + nt * 16 + l16);
             const uint32_t j  = c / P.tq, t = t0 + c % P.tq;
             float *op = P.out + (((size_t)s * P.n_tok + t) * P.n_head_q + kvh * P.kv_mul + j) * HD;
 #pragma unroll
@@ -669,40 +603,6 @@ PrefillExtPlan prefill_ext_plan(uint32_t n_seq, uint32_t n_tok, uint32_t pos_0, 
     return pl;
 }
 
-/* Columns per wave (16 nt) and key groups for head_dim 128.  nt = 2 with one
- * group has the least work per score; where its workgroups are too few for the
- * CUs, narrower tiles and two groups make shorter chains of steps.  Measured on
- * MI355X, 16q/4kv gated, us (nt, groups: 2,1 / 2,2 / 1,2):
- *   sequences x tokens     2,1    2,2    1,2
- *        1 x   16          6.4    7.8    6.8   nothing to share: the keys are one block
- *        1 x   64          8.0   10.3    6.9
- *        1 x  512         17.0   17.2   12.0
- *        1 x 1000         26.3   24.5   17.8
- *        2 x 1000         27.5   25.6   24.1   504 workgroups at nt 1
- *        4 x  512         18.8   19.1   18.9   512
- *        1 x 2500         57.6   47.6   54.0   316 at nt 2
- *        1 x 4096         93.9   83.3  110.8   512 at nt 2
- *        4 x 1000         31.0   36.1   45.7   512 at nt 2
- *        2 x 2500         64.5   77.0   95.2   632 at nt 2
- * A causal launch ends with its lightest tiles, so it may exceed a round of
- * workgroups (one of two groups a CU).  A sliding-window layer keeps one group:
- * its rows are the same bits whatever the tiles per workgroup (window 256, 1 x
- * 1000: 14.4 us, 10.9 at nt 1 with two groups; 2 x 700 14.4 against 17.4). */
-struct PrefillSplit {
-    uint32_t nt, groups;
-};
-static PrefillSplit prefill_split(uint32_t n_seq, uint32_t n_tok, uint32_t pos_0, uint32_t window, uint32_t n_head_kv,
-                                  uint32_t kv_mul) {
-    auto wgs = [&](uint32_t nt) {
-        const uint32_t tq = 64u * nt / kv_mul;
-        return (uint64_t)((n_tok + tq - 1u) / tq) * n_head_kv * n_seq;
-    };
-    if (window || (uint64_t)pos_0 + n_tok < 64u) return {2u, 1u};
-    if (wgs(1u) <= 512u) return {1u, 2u};
-    if (wgs(2u) <= 512u && n_tok >= 2048u) return {2u, 2u};
-    return {2u, 1u};
-}
-
 bool prefill_ext_supports(uint32_t head_dim, uint32_t kv_mul) {
     return (head_dim == 128u || head_dim == 64u) && kv_mul >= 1u && kv_mul <= 32u && (128u % kv_mul) == 0u;
 }
@@ -737,21 +637,10 @@ int launch_prefill_ext(const float *q, const uint16_t *k, const uint16_t *v, con
     hipEvent_t ev0, ev1;
     profile_events(&ev0, &ev1);
     if (ev0) (void)hipEventRecord(ev0, stream);
-    const PrefillSplit sp = head_dim == 128u && pl.chain == 1u
-                                ? prefill_split(n_seq, n_tok, pos_0, window, n_head_kv, P.kv_mul)
-                                : PrefillSplit{2u, 1u};
-    if (sp.groups == 2u) {
-        P.tq       = 64u * sp.nt / P.kv_mul;
-        P.n_qtiles = (n_tok + P.tq - 1u) / P.tq;
-        P.n_light  = 0u;
-        const dim3 grid(P.n_qtiles * n_head_kv * n_seq);
-        if (sp.nt == 1u) hipLaunchKernelGGL((k_prefill_ext<128, 1, 2>), grid, dim3(512), 0, stream, P);
-        else hipLaunchKernelGGL((k_prefill_ext<128, 2, 2>), grid, dim3(512), 0, stream, P);
-    } else if (head_dim == 128u) {
-        hipLaunchKernelGGL((k_prefill_ext<128, 2, 1>), dim3(n_wg), dim3(256), 0, stream, P);
-    } else {
-        hipLaunchKernelGGL((k_prefill_ext<64, 2, 1>), dim3(n_wg), dim3(256), 0, stream, P);
-    }
+    if (head_dim == 128u)
+        hipLaunchKernelGGL(k_prefill_ext<128>, dim3(n_wg), dim3(256), 0, stream, P);
+    else
+        hipLaunchKernelGGL(k_prefill_ext<64>, dim3(n_wg), dim3(256), 0, stream, P);
     hipError_t e = hipGetLastError();
     if (ev1) (void)hipEventRecord(ev1, stream);
     return hip_status(e);

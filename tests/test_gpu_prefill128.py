@@ -102,21 +102,21 @@ def test_prefill128_window_vs_oracle(gpu, orc, n_tok, pos_0, window, kv_pos0):
 
 
 @pytest.mark.parametrize("n_seq,n_tok,pos_0,window,kv_pos0,nq,nkv", [
-    (1, 63, 0, 0, 0, 16, 4),       # one group of waves
-    (1, 64, 0, 0, 0, 16, 4),       # two groups at 16 columns; the first tiles leave the second none
+    (1, 63, 0, 0, 0, 16, 4),       # two key blocks, the second short
+    (1, 64, 0, 0, 0, 16, 4),
     (1, 1, 63, 0, 0, 8, 8),        # one row
-    (1, 33, 31, 1, 31, 16, 4),     # a window: one group
-    (2, 130, 77, 0, 0, 32, 1),     # kv_mul 32: tiles of two rows
+    (1, 33, 31, 1, 31, 16, 4),     # window 1, the buffer starts at the first row
+    (2, 130, 77, 0, 0, 32, 1),     # kv_mul 32: tiles of four rows
     (1, 1001, 5, 256, 0, 16, 4),   # a window, ragged
-    (2, 1024, 0, 0, 0, 16, 4),     # the last size at 16 columns (512 workgroups) ...
-    (2, 1025, 0, 0, 0, 16, 4),     # ... and one group after it
-    (1, 2049, 300, 0, 0, 16, 4),   # two groups at 32 columns
-    (3, 1370, 2, 0, 0, 16, 4),     # one group
+    (2, 1024, 0, 0, 0, 16, 4),     # 256 workgroups ...
+    (2, 1025, 0, 0, 0, 16, 4),     # ... and 264, ragged
+    (1, 2049, 300, 0, 0, 16, 4),
+    (3, 1370, 2, 0, 0, 16, 4),     # 516: more than one round
 ])
 def test_prefill128_tile_shapes(gpu, orc, n_seq, n_tok, pos_0, window, kv_pos0, nq, nkv):
-    """Each tile width and group count of the launch, at the sizes where one
-    gives way to the next: rows at the edges of 32-key blocks and of the tiles
-    against the oracle (same tolerance as every prefill)."""
+    """Ragged sizes and workgroup counts around a round of the chip: rows at the
+    edges of 32-key blocks and of the tiles against the oracle (same tolerance as
+    every prefill)."""
     rng = np.random.default_rng(n_tok + pos_0 + window)
     q, k16, v16, g, got = run(gpu, rng, n_seq, n_tok, pos_0, nq, nkv, window=window, kv_pos0=kv_pos0)
     rows = sorted({r for e in (0, 16, 32, 64, 256, 640, n_tok) for r in (e - 1, e) if 0 <= r < n_tok})
@@ -125,6 +125,43 @@ def test_prefill128_tile_shapes(gpu, orc, n_seq, n_tok, pos_0, window, kv_pos0, 
         parity(got[s][rows], want, what=f"prefill128 tiles s={s} n={n_tok} pos0={pos_0} window={window}")
     vmax = np.abs(f16_to_f32(v16)).max()
     assert np.all(np.isfinite(got)) and np.abs(got).max() <= vmax + 1e-3
+
+
+@pytest.mark.parametrize("pattern", ["plain", "rising", "spike", "sunk"])
+@pytest.mark.parametrize("window", [0, 200])
+@pytest.mark.parametrize("nq,nkv", [(16, 4), (8, 8)])
+def test_prefill128_row_bits_do_not_depend_on_the_call(gpu, orc, pattern, window, nq, nkv):
+    """A prompt alone and among eight, whole and in two pieces: every row the
+    same bits; the rows of the first call within tolerance of the oracle.  Keys
+    that share a direction with every query give scores that climb, are huge on
+    single keys, or lie below -128 log2 units in the first block."""
+    la = gpu
+    rng = np.random.default_rng(nq + window)
+    n_tok, cut = 600, 230
+    q = rng.standard_normal((1, n_tok, nq, HD), dtype=np.float32)
+    k = rng.standard_normal((1, n_tok, nkv, HD), dtype=np.float32) * np.float32(0.5)
+    if pattern != "plain":
+        u = rng.standard_normal(HD).astype(np.float32)
+        u /= np.linalg.norm(u)
+        q += 3.0 * u
+        t = np.arange(n_tok, dtype=np.float32)
+        amp = {"rising": 0.25 * t, "spike": np.where(t % 97 == 40, 60.0, 0.0), "sunk": np.where(t < 32, -400.0, 0.0)}
+        k += amp[pattern].astype(np.float32)[None, :, None, None] * u
+    k16, v16 = f16(k), f16(rng.standard_normal((1, n_tok, nkv, HD), dtype=np.float32))
+    gate = rng.standard_normal((1, n_tok, nq)).astype(np.float32)
+
+    def call(n_seq, lo, hi):
+        rep = lambda x, a, b: np.broadcast_to(x[:, a:b], (n_seq, b - a, *x.shape[2:]))  # noqa: E731
+        return run(la, rng, n_seq, hi - lo, lo, nq, nkv, window=window, q=rep(q, lo, hi), k16=rep(k16, 0, hi),
+                   v16=rep(v16, 0, hi), gate_values=rep(gate, lo, hi))[-1]
+
+    one = call(1, 0, n_tok)[0]
+    rows = [0, 1, 31, 32, 33, 199, 200, 229, 230, 320, 511, 599]
+    want = oracle(orc, q, k16, v16, gate, 0, 0, 0, window, nq, nkv, rows=rows)
+    parity(one[rows], want, what=f"prefill128 {pattern} window={window} {nq}q/{nkv}kv")
+    for n_seq, lo, hi in ((8, 0, n_tok), (1, 0, cut), (8, 0, cut), (1, cut, n_tok), (8, cut, n_tok)):
+        got = call(n_seq, lo, hi)
+        assert np.all(got.view(np.uint32) == one[lo:hi].view(np.uint32)), f"{n_seq} sequences, rows {lo}..{hi}"
 
 
 def test_prefill128_lfm3_full_size_sampled(gpu, orc):
