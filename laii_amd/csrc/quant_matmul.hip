@@ -560,7 +560,9 @@ hipError_t launch_tokens(const MatSet &S, const void *x_q8, uint32_t nb, uint32_
  * is the reference's integer sum.  Sums over bsums (Q4_K and Q5_K mins, Q6_K
  * offsets) are one v_mfma_f32_16x16x32_f16 on each bsum's low byte and its
  * high byte times 256 (both exact in fp16): exact while the sum stays below
- * 2^24, which any block of int8 activations does.  The 32-weight block types
+ * 2^24, which bsums of -2048..2047 keep (16 x 2048 x 128 = 2^22); no 16 int8
+ * values sum to others, and a tile with such a bsum takes the dot4 kernel's
+ * integer sums.  The 32-weight block types
  * (Q4_0, Q8_0) need their int sum per block, one v_mfma_i32_16x16x32_i8 each,
  * started from kMagic, whose bits read as a float are 1.5 * 2^23 + sum: then
  *   fma(d, that float, -d * 1.5 * 2^23) = d * sum, rounded once (d * 1.5 * 2^23
@@ -592,6 +594,9 @@ __device__ __forceinline__ float sub_rounded(float a, float b) {
 
 __device__ __forceinline__ uint32_t pk_mul(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, (u16x2_t)(__builtin_bit_cast(u16x2_t, a) * __builtin_bit_cast(u16x2_t, b)));
+}
+__device__ __forceinline__ uint32_t pk_add(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, (u16x2_t)(__builtin_bit_cast(u16x2_t, a) + __builtin_bit_cast(u16x2_t, b)));
 }
 __device__ __forceinline__ uint32_t pk_mad(uint32_t a, uint32_t b, uint32_t c) {
     return __builtin_bit_cast(uint32_t, (u16x2_t)(__builtin_bit_cast(u16x2_t, a) * __builtin_bit_cast(u16x2_t, b) +
@@ -951,6 +956,7 @@ template <int TYPE, uint32_t NTOK, uint32_t THREADS> struct XStage {
     u32x4_t v[N], bv[NB ? NB : 1];
     uint32_t cv[NC ? NC : 1], off[N], boff[NB ? NB : 1], coff[NC ? NC : 1], doff;
     float d;
+    uint64_t wide = 0; /* lanes of this wave that staged a bsum outside -2048..2047 (in SGPRs: the registers are full) */
     const uint8_t *base;
     uint32_t tid;
 
@@ -1007,6 +1013,17 @@ template <int TYPE, uint32_t NTOK, uint32_t THREADS> struct XStage {
                 kMagic - 8 * ((int32_t)(int16_t)(cv[i] & 0xFFFFu) + (int32_t)(int16_t)(cv[i] >> 16));
         }
         if (tid < NTOK) X.d8[tid] = d;
+    }
+    /* the bsums just staged (not between put and the barrier, where the other
+     * waves would wait for it too) */
+    __device__ __forceinline__ void check() {
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i) {
+            uint32_t m = 0; /* bits 12..15 of each half of bsum + 2048: outside the range */
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) m |= pk_add(bv[i][j], 0x08000800u);
+            wide |= __builtin_amdgcn_ballot_w64((m & 0xF000F000u) != 0u);
+        }
     }
 };
 
@@ -1081,7 +1098,7 @@ __device__ __forceinline__ i32x4_t magic_splat() {
 
 /* a row and token at a time: rows whose scales are not all finite, where a
  * super-block whose d8 is 0 must be left out (elsewhere its term is a zero,
- * which changes no sum) */
+ * which changes no sum), and tokens whose bsums are not sums of int8 values */
 template <int TYPE>
 __device__ __noinline__ void slow_rows(const uint8_t *w, float *out, uint32_t n_rows, uint32_t r0, uint32_t r1,
                                        const uint8_t *xq, uint32_t nb, uint32_t n_tokens, uint32_t t0, uint32_t t1) {
@@ -1129,6 +1146,7 @@ __device__ __forceinline__ void few_tile(const uint8_t *__restrict__ w, float *_
             if (c0 + k >= nb) break;
             ws[u].put(mine.w);
             xs[u].put(mine.x);
+            xs[u].check();
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier(); /* the image is this wave's own */
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1154,7 +1172,7 @@ __device__ __forceinline__ void few_tile(const uint8_t *__restrict__ w, float *_
         for (uint32_t k = 0; k < n_k; ++k) sumf = add_rounded(sumf, S.terms[k][tid]);
         __syncthreads();
     }
-    if (__syncthreads_or(bad)) {
+    if (__syncthreads_or(bad || (xs[0].wide | xs[1].wide) != 0u)) {
         slow_rows<TYPE>(w, out, n_rows, r0 + 4u * wave, r0 + 4u * wave + 4u, xq, nb, n_tokens, t0, t0 + 16u);
         return;
     }
@@ -1172,6 +1190,7 @@ __device__ __forceinline__ void few_tile(const uint8_t *__restrict__ w, float *_
 template <int TYPE, uint32_t T> struct ManyShared {
     XTile<TYPE, 16u * T> x;
     WTile<TYPE, 64u> w;
+    uint32_t wide[4]; /* per wave: it staged a bsum that is no sum of int8 values */
 };
 
 template <int TYPE, uint32_t T>
@@ -1194,8 +1213,13 @@ __device__ __forceinline__ void many_tile(const uint8_t *__restrict__ w, float *
         if (b) __syncthreads(); /* the last super-block's reads are done */
         ws.put(S.w);
         xs.put(S.x);
+        if (kHasBsums<TYPE> && b + 1u == nb) { /* every wave's finding, without a barrier of its own */
+            xs.check();
+            S.wide[wave] = xs.wide != 0u; /* the same from every lane */
+        }
         __syncthreads();
         if (b + 1u < nb) {
+            xs.check();
             ws.fetch(b + 1u);
             xs.fetch(b + 1u);
         }
@@ -1229,6 +1253,7 @@ __device__ __forceinline__ void many_tile(const uint8_t *__restrict__ w, float *
         }
     }
     const uint32_t rw = r0 + 16u * wave, row = rw + l16;
+    if constexpr (kHasBsums<TYPE>) bad |= (S.wide[0] | S.wide[1] | S.wide[2] | S.wide[3]) != 0u;
     if (__any(bad)) {
         slow_rows<TYPE>(w, out, n_rows, rw, rw + 16u, xq, nb, n_tokens, t0, t0 + 16u * T);
         return;

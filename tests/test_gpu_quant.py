@@ -280,3 +280,53 @@ def test_matrix_pipe_row_scale_not_finite(gpu, orc, qtype, n_rows, B):
     want = orc.matmul_q(w, qtype, np.ascontiguousarray(xq[pick]), n_cols)
     assert np.array_equal(out.numpy()[pick], want, equal_nan=True)
     assert np.isfinite(want[::2, 3]).all()
+
+
+def wide_bsums(rng, w, xq, qtype, tokens):
+    """Rows with their largest mins or offsets, and blocks whose bsums are not the
+    sums of their activations: sums past 2^24, which fp32 does not hold."""
+    blk = w.reshape(-1, {12: 144, 13: 176, 14: 210}[qtype])
+    if qtype == 14:
+        blk[::2, 192:208] = rng.integers(64, 128, (blk[::2].shape[0], 16))
+    else:
+        blk[::2, 4:16] = 0xFF
+    nb = xq.shape[1] // 292
+    for t in tokens:
+        b = int(rng.integers(nb))
+        xq[t, 292 * b + 260:292 * (b + 1)] = rng.integers(20000, 24000, 16).astype(np.int16).view(np.uint8)
+
+
+@pytest.mark.parametrize("qtype", [12, 13, 14])
+@pytest.mark.parametrize("n_rows,n_cols,B", [(5, 768, 5), (1000, 768, 270), (2050, 256, 260), (2060, 512, 1030)])
+def test_matrix_pipe_any_bsums(gpu, orc, qtype, n_rows, n_cols, B):
+    """Bsums that no int8 activations give, in some tokens, over every tile
+    shape: their integer sums stay exact, as with one token."""
+    la = gpu
+    rng = np.random.default_rng(qtype * 10 + B)
+    w = q_random(rng, qtype, n_rows, n_cols)
+    xq = orc.quantize_q8_K(rng.standard_normal((B, n_cols)).astype(np.float32))
+    odd = sorted({1, 3, B // 2, B - 1})
+    wide_bsums(rng, w, xq, qtype, odd)
+    out = la.DeviceArray.zeros((B, n_rows), np.float32)
+    la.matmul_prequant(out, dev(la, w), qtype, n_rows, n_cols, dev(la, xq), B)
+    pick = sorted({*odd, 0, 2, B // 3, B - 2})
+    want = orc.matmul_q(w, qtype, np.ascontiguousarray(xq[pick]), n_cols)
+    assert np.array_equal(out.numpy()[pick].view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("B", [9, 270, 1030])
+def test_matrix_pipe_any_bsums_mixed_set(gpu, orc, B):
+    """The same in a set of several types, one launch."""
+    la = gpu
+    rng = np.random.default_rng(B)
+    n_cols, rows, types = 512, [600, 300, 100, 40], [12, 14, 13, 8]
+    ws = [q_random(rng, t, r, n_cols) for t, r in zip(types, rows)]
+    xq = orc.quantize_q8_K(rng.standard_normal((B, n_cols)).astype(np.float32))
+    for w, t in zip(ws[:3], types):
+        wide_bsums(rng, w, xq, t, [2, B - 2])
+    outs = [la.DeviceArray.zeros((B, r), np.float32) for r in rows]
+    la.gqa_qkv_fused(outs, [dev(la, w) for w in ws], types, rows, n_cols, dev(la, xq), B)
+    pick = [0, 1, 2, 3, B // 2, B - 2, B - 1]
+    for o, w, t in zip(outs, ws, types):
+        want = orc.matmul_q(w, t, np.ascontiguousarray(xq[pick]), n_cols)
+        assert np.array_equal(o.numpy()[pick].view(np.uint32), want.view(np.uint32)), t
