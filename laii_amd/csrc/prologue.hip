@@ -421,9 +421,9 @@ int launch_qkv_prologue(float *q, const float *k, const float *v, uint16_t *cons
                      n_rows, n_head_q, n_head_kv, head_dim, window_len, cap, eps, prologue};
     if (head_dim == 64u || head_dim == 128u) {
         const uint32_t n_groups = (n_head_q + n_head_kv + 7u) / 8u;
-        const uint64_t units    = (uint64_t)n_groups * n_rows;
-        if (units <= 0xFFFFFFFCull) {
-            const dim3 grid((uint32_t)((units + 3u) / 4u), 1, n_seq);
+        const uint64_t blocks   = ((uint64_t)n_groups * n_rows + 3u) / 4u;
+        if (blocks * 256u <= 0xFFFFFFFFull) { /* a launch dimension holds 2^32 threads */
+            const dim3 grid((uint32_t)blocks, 1, n_seq);
             const bool table = prologue == LFM_PROLOGUE_TABLE;
             if (head_dim == 64u && table)
                 hipLaunchKernelGGL((k_qkv_prologue_wide<64, true>), grid, dim3(256), 0, stream, P, n_groups);
