@@ -163,9 +163,9 @@ class FusedStepWorkload(DecodeWorkload):
 
 def bench_engine_step(la, rng, nq=16, nkv=8, hd=64, pos=1023, calls=500):
     """lfm_attn_ctx_forward end to end, as the engine calls it per attention
-    layer (host q/k/v in, host output out, synchronous): one host-to-device
-    copy, the fused attention launch (+ split merge), one device-to-host
-    copy.  Config 1's shape (16q/8kv d64, position 1023).  Wall clock per
+    layer (host q/k/v in, host output out, synchronous): a kernel that reads
+    the inputs from pinned memory, the fused attention launch (+ split merge),
+    which writes its output there.  Config 1's shape (16q/8kv d64, position 1023).  Wall clock per
     call, median of 5 batches of `calls`."""
     ctx = la.EngineContext(1, nq, nkv, hd, pos + 1, 1e-5, rope_base=1e6)
     try:

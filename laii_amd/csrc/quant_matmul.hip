@@ -1306,7 +1306,7 @@ __global__ __launch_bounds__(256, 2) void k_matmul_mfma(const MatSet S, const ui
     case 14u: mfma_tile<14, T>(S, m, bx, xq, nb, n_tokens, sh); break;
     case 13u: mfma_tile<13, T>(S, m, bx, xq, nb, n_tokens, sh); break;
     case 23u: mfma_tile<23, T>(S, m, bx, xq, nb, n_tokens, sh); break;
-    case 2u:
+    case 2u: /* launch_mfma takes T = 8 for sets without Q4_0 only */
         if constexpr (T <= 4u) mfma_tile<2, T>(S, m, bx, xq, nb, n_tokens, sh);
         break;
     default: mfma_tile<8, T>(S, m, bx, xq, nb, n_tokens, sh); break;
@@ -1324,8 +1324,12 @@ hipError_t launch_tiles(MatSet S, const void *x_q8, uint32_t nb, uint32_t n_toke
 }
 
 /* Five or more tokens.  Measured on MI355X, us per call over 2048 columns:
- *  - few_tile while its 16 x 16 tiles make one round (four workgroups a CU):
- *    128 tokens x 2048 rows Q4_K 9.1, T = 2 9.8; x 3072 rows 11.8 against 9.9;
+ *  - few_tile up to 1024 of its 16 x 16 tiles, against T = 2.  A CU holds three
+ *    such workgroups (133 to 166 registers; Q6_K, Q8_0 and mixed sets also by
+ *    LDS), so 768 are a round and 1024 a round and a third: 128 tokens x 2048
+ *    rows Q4_K 9.1 against 9.9, Q5_K 11.3 / 12.1, Q6_K 12.6 / 14.3, IQ4_XS 11.4
+ *    / 12.7, Q4_0 9.9 / 11.5, Q8_0 10.3 / 11.7, a mixed set 12.4 / 14.6; two
+ *    whole rounds, x 3072 rows, Q4_K 11.8 against 9.9;
  *  - T = 2 while a CU gets at most one such workgroup: 256 x 2048 10.1, T = 4
  *    13.4; 700 x 2048 (704 workgroups) Q6_K 27.1 against 26.9, IQ4_XS 25.3
  *    against 22.8;

@@ -181,8 +181,8 @@ def test_other_types_bit_exact(gpu, orc, qtype, n_rows, n_cols, B):
 @pytest.mark.parametrize("B", [3, 9])
 def test_fused_mixed_types(gpu, orc, B):
     """One fused call over four matrices of four different types (Q5_K Q,
-    IQ4_XS K, Q8_0 V, Q4_0 gate); at 9 tokens the Q5_K matrix takes the
-    int8-MFMA kernel and the rest one dot4 launch."""
+    IQ4_XS K, Q8_0 V, Q4_0 gate), one launch: of the dot4 kernel up to four
+    tokens, on the matrix pipe at 9."""
     la = gpu
     rng = np.random.default_rng(99 + B)
     n_cols, rows, types = 2048, [2048, 512, 512, 16], [13, 23, 8, 2]
@@ -330,3 +330,56 @@ def test_matrix_pipe_any_bsums_mixed_set(gpu, orc, B):
     for o, w, t in zip(outs, ws, types):
         want = orc.matmul_q(w, t, np.ascontiguousarray(xq[pick]), n_cols)
         assert np.array_equal(o.numpy()[pick].view(np.uint32), want.view(np.uint32)), t
+
+
+@pytest.mark.parametrize("qtype", [2, 8, 12, 13, 14, 23])
+@pytest.mark.parametrize("n_rows,n_cols,B", [(20, 512, 6), (1000, 512, 270), (2050, 256, 260), (2060, 512, 1030)])
+@pytest.mark.parametrize("bits", [0x7C00, 0xFC00, 0x7E00])
+def test_matrix_pipe_scale_not_finite_every_tile(gpu, orc, qtype, n_rows, n_cols, B, bits):
+    """An infinite or NaN scale in the last block of one row and, where the type
+    has one, an infinite or NaN min scale in another, over every tile shape:
+    zero activation blocks are left out, the rows beside are untouched."""
+    la = gpu
+    rng = np.random.default_rng(qtype + B)
+    w = q_random(rng, qtype, n_rows, n_cols)
+    size = {2: 18, 8: 34, 12: 144, 13: 176, 14: 210, 23: 136}[qtype]
+    at = w.shape[1] - size + (208 if qtype == 14 else 0)
+    h = np.array([bits], np.uint16).view(np.uint8)
+    w[3, at:at + 2] = h
+    if qtype in (12, 13):
+        w[n_rows - 2, 2:4] = h
+    x = rng.standard_normal((B, n_cols)).astype(np.float32)
+    x[::2, -256:] = 0.0
+    x[::3, :256] = 0.0
+    xq = orc.quantize_q8_K(x)
+    out = la.DeviceArray.zeros((B, n_rows), np.float32)
+    la.matmul_prequant(out, dev(la, w), qtype, n_rows, n_cols, dev(la, xq), B)
+    pick = sorted({*range(min(B, 6)), B // 2, B - 2, B - 1})
+    want = orc.matmul_q(w, qtype, np.ascontiguousarray(xq[pick]), n_cols)
+    got = out.numpy()[pick]
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32))
+    assert np.isfinite(want[0::2, 3][: 2]).all() and not np.isfinite(want[1, 3])
+
+
+@pytest.mark.parametrize("B", [9, 270, 1030])
+def test_matrix_pipe_scale_not_finite_mixed_set(gpu, orc, B):
+    """The same in a set of several types, one launch."""
+    la = gpu
+    rng = np.random.default_rng(B + 1)
+    n_cols, rows, types = 512, [600, 300, 100, 40], [12, 14, 13, 8]
+    ws = [q_random(rng, t, r, n_cols) for t, r in zip(types, rows)]
+    inf = np.array([0x7C00], np.uint16).view(np.uint8)
+    ws[0][5, 2:4] = inf
+    ws[1][299, 208:210] = inf
+    ws[3][39, 34 * 5:34 * 5 + 2] = inf
+    x = rng.standard_normal((B, n_cols)).astype(np.float32)
+    x[::2, :256] = 0.0
+    xq = orc.quantize_q8_K(x)
+    outs = [la.DeviceArray.zeros((B, r), np.float32) for r in rows]
+    la.gqa_qkv_fused(outs, [dev(la, w) for w in ws], types, rows, n_cols, dev(la, xq), B)
+    pick = [0, 1, 2, 3, B // 2, B - 2, B - 1]
+    for o, w, t in zip(outs, ws, types):
+        want = orc.matmul_q(w, t, np.ascontiguousarray(xq[pick]), n_cols)
+        assert np.array_equal(o.numpy()[pick], want, equal_nan=True), t
