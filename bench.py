@@ -188,7 +188,7 @@ def bench_engine_step(la, rng, nq=16, nkv=8, hd=64, pos=1023, calls=500):
         ctx.close()
     us = float(np.median(per)) * 1e6
     return dict(us_per_call=round(us, 2), shape=f"{nq}q/{nkv}kv d{hd}, position {pos}, one layer",
-                includes="host->device copy, fused QK-norm+RoPE+K/V store+attention, merge, device->host copy, sync")
+                includes="inputs from pinned memory, fused QK-norm+RoPE+K/V store+attention, merge, output to pinned memory, sync")
 
 
 class PrefillWorkload:
